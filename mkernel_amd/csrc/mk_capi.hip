@@ -140,6 +140,31 @@ int check_ws(const void* ws, int64_t bytes, const char* fn) {
   return MK_OK;
 }
 
+constexpr int kNoSmallPlan = 1 << 30;
+
+// C = A @ B by the small-tile kernel (kNoSmallPlan: none of its tiles fits).
+int small_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+               int64_t ldc, void* ws, int64_t ws_bytes, int cus, void* stream, const char* where) {
+  mk::GemmSmallPlan plan;
+  if (!mk::plan_gemm_small(M, N, K, lda, ldb, cus, ws != nullptr, ws_bytes - kSplitFlagBytes, (int)(kClaimOffset / 4),
+                           &plan))
+    return kNoSmallPlan;
+  mk::GemmSmallParams p;
+  p.A = static_cast<const uint16_t*>(A);
+  p.B = static_cast<const uint16_t*>(B);
+  p.C = static_cast<uint16_t*>(C);
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.K = (int)K;
+  p.tiles_m = (int)(M / plan.bm);
+  p.tiles_n = (int)(N / plan.bn);
+  p.group_m = 8;
+  p.nk = (int)((K + 63) / 64);
+  p.words = static_cast<uint32_t*>(ws);
+  p.ws = ws ? reinterpret_cast<float*>(static_cast<char*>(ws) + kSplitFlagBytes) : nullptr;
+  hipError_t e = mk::launch_gemm_small(p, plan, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MK_OK : hip_fail(e, where);
+}
+
 // num_producers <= -3 asks for the co-resident staging kernel with
 // -2 - num_producers one-wave workgroups per CU (1..4).  Under graph capture
 // the fork/join would become two graph branches whose order the replay does
@@ -263,10 +288,10 @@ int mk_gemm(const mk_gemm_args* a, void* stream) {
   int bm = a->tile_m;
   if (bm == 0) {
     // 256-row tiles unless 128-row ones fit in one round: a partial round
-    // of 256-row tiles (spread over the XCDs) beats two rounds of 128-row
-    // ones (4352x2048x8192: 137 vs 176 us; 4096x3584x8192: 188 vs 264 us),
-    // while one round of 128-row tiles beats a half-empty 256-row round
-    // (4096x2048x8192: 137 vs 145 us; 2048^2 x 8192: 116 vs 128 us).
+    // of 256-row tiles (spread over the XCDs) beats two rounds of smaller
+    // ones (4096x3584x8192: 188 us, 128 x 256 tiles of the small-tile kernel
+    // 233, of this kernel 264), while a half-empty 256-row round loses to
+    // one round of smaller tiles (2048x2048x8192: 128 us against 76).
     const int64_t t256 = (a->M % 256 == 0) ? (a->M / 256) * (a->N / 256) : 0;
     bm = (2 * t256 > d.cus) ? 256 : 128;
   }
@@ -277,6 +302,17 @@ int mk_gemm(const mk_gemm_args* a, void* stream) {
     return fail(MK_ESHAPE, "mk_gemm: leading dimensions must cover the row and be multiples of 8");
   if (!aligned16(a->A) || !aligned16(a->B) || !aligned16(a->C))
     return fail(MK_EINVAL, "mk_gemm: pointers must be 16-byte aligned");
+  if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm")) return rc;
+  int total;
+  if (int rc = grid_total(a->num_cus, d, "mk_gemm", &total)) return rc;
+  // Less than a round of 256-row tiles: the small-tile kernel.  A call that
+  // names a tile height, a wave count or a grid keeps the persistent kernel,
+  // whose arguments those are.
+  if (bm == 128 && a->tile_m == 0 && a->waves == 0 && a->num_cus == 0) {
+    const int rc = small_gemm(a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc, a->split_ws,
+                              a->split_ws_bytes, d.cus, stream, "mk_gemm launch");
+    if (rc != kNoSmallPlan) return rc;
+  }
   mk::GemmKParams p;
   fill_common(p);
   p.A = static_cast<const uint16_t*>(a->A);
@@ -286,11 +322,8 @@ int mk_gemm(const mk_gemm_args* a, void* stream) {
   p.M = (int)a->M; p.N = (int)a->N; p.K = (int)a->K;
   p.tiles_m = (int)(a->M / bm);
   p.tiles_n = (int)(a->N / 256);
-  int total;
-  if (int rc = grid_total(a->num_cus, d, "mk_gemm", &total)) return rc;
   set_grid(p, total, 0, p.tiles_m * p.tiles_n);
   if (a->waves) p.waves = a->waves;
-  if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm")) return rc;
   plan_split(p, bm, a->split_ws, a->split_ws_bytes);
   hipError_t e = mk::launch_gemm(p, bm, mk::kEpiStore, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? MK_OK : hip_fail(e, "mk_gemm launch");

@@ -104,6 +104,28 @@ hipError_t launch_gemm(const GemmKParams& p, int bm, int epi, hipStream_t stream
 hipError_t launch_gemm_costaged(const GemmKParams& p, int epi, int n_stage_waves, hipStream_t stream);
 hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream);
 
+// Dense GEMM of less than one round of persistent tiles (mk_gemm_small.hip).
+struct GemmSmallParams {
+  const uint16_t* A;
+  const uint16_t* B;
+  uint16_t* C;
+  int64_t lda, ldb, ldc;
+  int K;
+  int tiles_m, tiles_n, group_m;
+  int nk;            // 64-deep K stages of a tile
+  uint32_t* words;   // a ticket per tile and a header per workgroup, zero between launches
+  float* ws;         // an fp32 tile per workgroup
+};
+struct GemmSmallPlan {
+  int tile, bm, bn;  // index into the kernel's tile table, and its shape
+  int grid, split;   // workgroups, and parts of each tile along K
+};
+// The tile and split with the least estimated time; false: no tile fits.
+// ws: a workspace of ws_words words and ws_tiles_bytes of tiles is there.
+bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int cus, bool ws, int64_t ws_tiles_bytes,
+                     int ws_words, GemmSmallPlan* plan);
+hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, hipStream_t stream);
+
 struct PermuteKParams {
   const uint16_t* tokens;
   const int* pull;
