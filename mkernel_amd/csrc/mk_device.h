@@ -98,14 +98,18 @@ __device__ __forceinline__ void wait_vmem_all() { __builtin_amdgcn_s_waitcnt(0x0
 // (buffer_wbl2), which is only needed for data written without SC1 — and
 // that write-back flushes every dirty line of the XCD's L2, which cost the
 // staging ~15 % of the launch when it ran once per published batch.
+// What is left after the whole batches goes as one more batch whose loads and
+// stores run through buffer descriptors of the copied range: lanes past the
+// end load nothing and store nothing.  (A loop of single loads there made a
+// copy of less than a batch serial: 102 KB pieces took 25 load latencies.)
 template <int NT, int U>
 __device__ __forceinline__ void copy_wt(const void* src, void* dst, int64_t nvec) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const u32x4* s = static_cast<const u32x4*>(src);
   const __amdgpu_buffer_rsrc_t r = make_rsrc(dst, (uint32_t)(nvec * 16));
-  constexpr int kCpolSc1 = 0x10;  // gfx940+ cache policy: SC1
+  constexpr int kCpolNt = 0x2, kCpolSc1 = 0x10;  // gfx940+ cache policy: nontemporal, SC1
   int64_t base = threadIdx.x;
-  for (; base + (int64_t)(U - 1) * NT < nvec; base += (int64_t)U * NT) {
+  for (; base - threadIdx.x + U * NT <= nvec; base += U * NT) {
     u32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(s + base + u * NT);
@@ -113,8 +117,16 @@ __device__ __forceinline__ void copy_wt(const void* src, void* dst, int64_t nvec
     for (int u = 0; u < U; ++u)
       __builtin_amdgcn_raw_buffer_store_b128(v[u], r, (int)((base + u * NT) * 16), 0, kCpolSc1);
   }
-  for (; base < nvec; base += NT)
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_nontemporal_load(s + base), r, (int)(base * 16), 0, kCpolSc1);
+  if (base - threadIdx.x < nvec) {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, (uint32_t)(nvec * 16));
+    u32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((base + u * NT) * 16), 0, kCpolNt));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      __builtin_amdgcn_raw_buffer_store_b128(v[u], r, (int)((base + u * NT) * 16), 0, kCpolSc1);
+  }
 }
 
 }  // namespace mk
