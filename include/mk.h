@@ -82,6 +82,10 @@ int mk_gemm(const mk_gemm_args* args, void* stream);
  *                            round while the other computes
  *   gated, producers == -2 : cooperative staging with every workgroup
  *                            copying an even share before every round
+ *                            (both: with num_cus == 0 the library may instead
+ *                            queue a copy kernel on every CU that stages and
+ *                            publishes all blocks, then the GEMM, where that
+ *                            is faster; same outputs, flags and counters)
  *   gated, producers <= -3 : wave-specialised producer: a staging kernel of
  *                            (-2 - producers) one-wave workgroups per
  *                            compute workgroup (1..4) runs beside a GEMM
@@ -171,7 +175,8 @@ typedef struct mk_gemm_rs_args {
   const int32_t* stage_order;   /* [(world-1) * (M/world)/128]; NULL = ascending */
   uint32_t epoch;
   int32_t gated;
-  int32_t num_producers;        /* as in mk_ag_gemm; -1 and -2 = cooperative staging, even share;
+  int32_t num_producers;        /* as in mk_ag_gemm; -1 and -2 = cooperative staging, even share
+                                   (or staged first by a copy kernel, with num_cus == 0);
                                    <= -3 = co-resident staging kernel (needs split_ws) */
   int32_t num_cus;
   uint32_t spin_limit;
@@ -216,7 +221,8 @@ typedef struct mk_gemm_ar_args {
   const int32_t* stage_order;   /* [(world-1) * M/128]; NULL = ascending, no arrival order */
   uint32_t epoch;
   int32_t gated;
-  int32_t num_producers;        /* as in mk_ag_gemm; -1 and -2 = cooperative staging, even share;
+  int32_t num_producers;        /* as in mk_ag_gemm; -1 and -2 = cooperative staging, even share
+                                   (or staged first by a copy kernel, with num_cus == 0);
                                    <= -3 = co-resident staging kernel (needs split_ws) */
   int32_t num_cus;
   uint32_t spin_limit;

@@ -114,8 +114,9 @@ constexpr int64_t kClaimOffset = kSplitFlagBytes - 64;
 int64_t split_ws_bytes(int cus) { return kSplitFlagBytes + (int64_t)cus * kSplitTileBytes; }
 
 // K-split plan for the tail round: with R = tiles % n_cons tiles left for a
-// partial last round, split each of them s = min(4, n_cons / R) ways along
-// K so that R*s workgroups share the round.  The workspace holds the flag
+// partial last round, split each of them s ways along K so that R*s workgroups
+// share the round: as many as fit, up to 4, for the expert GEMMs, which stream
+// weights; as tail_split finds best for dense 256-row tiles.  The workspace holds the flag
 // words at a fixed offset (so every plan finds them zeroed) followed by
 // R*(s-1) < n_cons <= CUs partial tiles, which split_ws_bytes covers.
 void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn = 256) {
@@ -125,6 +126,7 @@ void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn =
   if (p.perm_mode != mk::kPermNone && ntiles > mk::kMaxSplitListTiles) return;
   int s = std::min(4, p.n_cons / R);
   s = std::min(s, (p.K / 32) / 4);  // keep every part at >= 4 K stages
+  if (bm == 256) s = mk::tail_split(R, p.K, p.n_cons, nullptr);
   if (s < 2) return;
   const int64_t parts = (int64_t)R * (s - 1);
   if (parts * 4 > kClaimOffset || kSplitFlagBytes + parts * bm * bn * 4 > ws_bytes) return;
@@ -142,14 +144,10 @@ int check_ws(const void* ws, int64_t bytes, const char* fn) {
 
 constexpr int kNoSmallPlan = 1 << 30;
 
-// C = A @ B by the small-tile kernel (kNoSmallPlan: none of its tiles fits).
-int small_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-               int64_t ldc, void* ws, int64_t ws_bytes, int cus, void* stream, const char* where) {
-  mk::GemmSmallPlan plan;
-  if (!mk::plan_gemm_small(M, N, K, lda, ldb, cus, ws != nullptr, ws_bytes - kSplitFlagBytes, (int)(kClaimOffset / 4),
-                           &plan))
-    return kNoSmallPlan;
+mk::GemmSmallParams small_params(const mk::GemmSmallPlan& plan, const void* A, const void* B, void* C, int64_t M,
+                                 int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc) {
   mk::GemmSmallParams p;
+  std::memset(&p, 0, sizeof p);
   p.A = static_cast<const uint16_t*>(A);
   p.B = static_cast<const uint16_t*>(B);
   p.C = static_cast<uint16_t*>(C);
@@ -159,9 +157,88 @@ int small_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   p.tiles_n = (int)(N / plan.bn);
   p.group_m = 8;
   p.nk = (int)((K + 63) / 64);
-  p.words = static_cast<uint32_t*>(ws);
-  p.ws = ws ? reinterpret_cast<float*>(static_cast<char*>(ws) + kSplitFlagBytes) : nullptr;
-  hipError_t e = mk::launch_gemm_small(p, plan, static_cast<hipStream_t>(stream));
+  return p;
+}
+
+// C = A @ B by the small-tile kernel.  kNoSmallPlan: none of its tiles fits,
+// or the persistent kernel's 256-row tiles do and are estimated to be faster.
+int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
+  mk::GemmSmallPlan plan;
+  if (!mk::plan_gemm_small(a->M, a->N, a->K, a->lda, a->ldb, cus, a->split_ws != nullptr,
+                           a->split_ws_bytes - kSplitFlagBytes, (int)(kClaimOffset / 4), {-1, 0}, &plan))
+    return kNoSmallPlan;
+  const int64_t t256 = a->M % 256 ? 0 : (a->M / 256) * (a->N / 256);
+  if (2 * t256 > cus && mk::persistent_cost(t256, a->K, cus, a->split_ws != nullptr) <= plan.us) return kNoSmallPlan;
+  mk::GemmSmallParams p = small_params(plan, a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc);
+  p.words = static_cast<uint32_t*>(a->split_ws);
+  if (a->split_ws) p.ws = reinterpret_cast<float*>(static_cast<char*>(a->split_ws) + kSplitFlagBytes);
+  hipError_t e = mk::launch_gemm_small(p, plan, false, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MK_OK : hip_fail(e, "mk_gemm launch");
+}
+
+// A fused launch `p` as a sequence: the staging of its blocks on every CU, then
+// the small-tile kernel on whole tiles, then the done flags.  kNoSmallPlan: the
+// persistent kernel is to run; `p` then stages nothing any more if its blocks
+// were better staged first.  Every output is the same K-ordered sum on each
+// path (where the persistent kernel would split its tail along K it runs), so
+// results do not depend on how the blocks arrive.  Not for flags that someone
+// else publishes: those must be able to arrive while the launch waits.
+//
+// The persistent kernel's workgroups copy between their tiles, which hides
+// part of the copy behind others' tiles when there are several rounds and a
+// round is longer than its share of the copy.  Staging first was faster (us,
+// in the launch -> first) for AllGather below two rounds (12288x1280x2784 114
+// -> 100) or K 2048 (16384x3584x1024 146 -> 138; 16384x3584x8192 805 -> 812)
+// and for ReduceScatter below K 1024 (16384x8192, world 8: K 512 321 -> 233,
+// 1536 453 -> 449, 3584 865 -> 871); the all-reduces, whose fold or second
+// copy is spread over all rounds, gained nothing (8192^2, two-shot, K 768 171
+// -> 179).  The tiles of the persistent kernel are too large where there are
+// few (AllGather 4096x256x4096, world 16: 211 -> 32 with the small ones) and
+// where few rows are folded by whole workgroups (ReduceScatter 4096x4096x256,
+// world 16: 69 -> 50).
+int small_fused(mk::GemmKParams& p, bool reduce, int cus, void* stream, const char* where) {
+  if (p.sk_split > 1) return kNoSmallPlan;
+  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+  mk::GemmSmallPlan plan;
+  const mk::SmallFold fold{reduce ? p.rs_npeers : -1, p.rs_own_rows};
+  bool small = mk::plan_gemm_small(p.M, p.N, p.K, p.lda, p.ldb, cus, false, 0, 0, fold, &plan);
+  if (small) {
+    double one = mk::persistent_cost(tiles, p.K, cus, false), sm = plan.us;
+    if (reduce) {
+      // a workgroup of the persistent kernel folds in about two of its rounds
+      // when the last is not full; either kernel moves its stores and partials
+      // at 2.5 TB/s at most
+      const double bytes = 2.0 * p.N * ((double)p.M + (double)p.rs_npeers * p.rs_own_rows) / 2.5e6;
+      const bool partial = tiles > cus && tiles % cus;
+      one += (partial ? 2.0 : 1.0) * mk::fold_cost(fold, (double)p.rs_own_rows / 256 * p.tiles_n, 65536.0, cus);
+      one = std::max(one, bytes) + (partial ? 14.0 : 7.0);
+      sm = std::max(sm, bytes) + 8.0;
+    }
+    small = sm < one;
+  }
+  const bool first = p.st_nblocks > 0 &&
+                     (small || (reduce ? p.K < 1024 && !p.st_src2 && p.rs_own_rows < p.M
+                                       : tiles < 2 * cus || p.K < 2048));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (first) {
+    hipError_t e = mk::launch_stage_all(p, std::min(p.st_nblocks * mk::kPieces, 8 * cus), s);
+    if (e != hipSuccess) return hip_fail(e, where);
+  }
+  if (!small) {
+    if (first) {
+      // the flags are published: the launch gates on them without a wait
+      p.st_nblocks = 0;
+      p.st_coop = 0;
+    }
+    return kNoSmallPlan;
+  }
+  mk::GemmSmallParams q = small_params(plan, p.A, p.B, p.C, p.M, p.N, p.K, p.lda, p.ldb, p.ldc);
+  q.rs_own_row0 = p.rs_own_row0; q.rs_own_rows = p.rs_own_rows; q.rs_npeers = p.rs_npeers;
+  q.rs_recv = p.rs_recv; q.rs_out = p.rs_out;
+  hipError_t e = mk::launch_gemm_small(q, plan, reduce, s);
+  if (e == hipSuccess && p.ar_done)
+    e = mk::launch_publish_done(p.ar_done + p.rs_own_row0 / 256 * p.tiles_n, p.rs_own_rows / 256 * p.tiles_n,
+                                p.epoch_ptr, p.epoch, s);
   return e == hipSuccess ? MK_OK : hip_fail(e, where);
 }
 
@@ -287,11 +364,8 @@ int mk_gemm(const mk_gemm_args* a, void* stream) {
   if (int rc = device_info(&d)) return rc;
   int bm = a->tile_m;
   if (bm == 0) {
-    // 256-row tiles unless 128-row ones fit in one round: a partial round
-    // of 256-row tiles (spread over the XCDs) beats two rounds of smaller
-    // ones (4096x3584x8192: 188 us, 128 x 256 tiles of the small-tile kernel
-    // 233, of this kernel 264), while a half-empty 256-row round loses to
-    // one round of smaller tiles (2048x2048x8192: 128 us against 76).
+    // 256-row tiles from half a round of them on (below, the small-tile
+    // kernel runs: 2048x2048x8192 76 us, 128 with 256-row tiles)
     const int64_t t256 = (a->M % 256 == 0) ? (a->M / 256) * (a->N / 256) : 0;
     bm = (2 * t256 > d.cus) ? 256 : 128;
   }
@@ -305,12 +379,10 @@ int mk_gemm(const mk_gemm_args* a, void* stream) {
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm")) return rc;
   int total;
   if (int rc = grid_total(a->num_cus, d, "mk_gemm", &total)) return rc;
-  // Less than a round of 256-row tiles: the small-tile kernel.  A call that
-  // names a tile height, a wave count or a grid keeps the persistent kernel,
-  // whose arguments those are.
-  if (bm == 128 && a->tile_m == 0 && a->waves == 0 && a->num_cus == 0) {
-    const int rc = small_gemm(a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc, a->split_ws,
-                              a->split_ws_bytes, d.cus, stream, "mk_gemm launch");
+  // A call that names a tile height, a wave count or a grid keeps the
+  // persistent kernel, whose arguments those are.
+  if (a->tile_m == 0 && a->waves == 0 && a->num_cus == 0) {
+    const int rc = small_gemm(a, d.cus, stream);
     if (rc != kNoSmallPlan) return rc;
   }
   mk::GemmKParams p;
@@ -335,7 +407,7 @@ namespace {
 // Validates mk_ag_gemm's arguments and fills the launch: every refusal
 // happens here, before anything is queued.  *costage_waves > 0 selects the
 // co-resident staging kernel (that many one-wave workgroups).
-int prepare_ag(const mk_ag_gemm_args* a, void* stream, mk::GemmKParams& p, int* costage_out) {
+int prepare_ag(const mk_ag_gemm_args* a, void* stream, mk::GemmKParams& p, int* costage_out, int* small_cus) {
   if (!a || !a->A_full || !a->B || !a->C) return fail(MK_EINVAL, "mk_ag_gemm: null argument");
   DevInfo d;
   if (int rc = device_info(&d)) return rc;
@@ -405,10 +477,16 @@ int prepare_ag(const mk_ag_gemm_args* a, void* stream, mk::GemmKParams& p, int* 
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_ag_gemm")) return rc;
   plan_split(p, bm, a->split_ws, a->split_ws_bytes);
   *costage_out = costage_waves * total;
+  // staged by this call, or not gated at all
+  *small_cus = (a->num_cus == 0 && (!a->gated || (coop && !costage_waves))) ? d.cus : 0;
   return MK_OK;
 }
 
-int launch_ag(const mk::GemmKParams& p, int costage, void* stream) {
+int launch_ag(mk::GemmKParams& p, int costage, int small_cus, void* stream) {
+  if (small_cus) {
+    const int rc = small_fused(p, false, small_cus, stream, "mk_ag_gemm launch");
+    if (rc != kNoSmallPlan) return rc;
+  }
   hipError_t e = costage ? mk::launch_gemm_costaged(p, mk::kEpiStore, costage, static_cast<hipStream_t>(stream))
                          : mk::launch_gemm(p, 256, mk::kEpiStore, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? MK_OK : hip_fail(e, "mk_ag_gemm launch");
@@ -419,9 +497,9 @@ extern "C" {
 
 int mk_ag_gemm(const mk_ag_gemm_args* a, void* stream) {
   mk::GemmKParams p;
-  int costage = 0;
-  if (int rc = prepare_ag(a, stream, p, &costage)) return rc;
-  return launch_ag(p, costage, stream);
+  int costage = 0, small_cus = 0;
+  if (int rc = prepare_ag(a, stream, p, &costage, &small_cus)) return rc;
+  return launch_ag(p, costage, small_cus, stream);
 }
 
 
@@ -446,8 +524,8 @@ int mk_ag_gemm_noalloc(const mk_ag_gemm_args* a, void* stream) {
   if (b.num_producers <= -3) b.num_producers = -1;
   // every argument check before anything is queued on the stream
   mk::GemmKParams p;
-  int costage = 0;
-  if (int rc = prepare_ag(&b, stream, p, &costage)) return rc;
+  int costage = 0, small_cus = 0;
+  if (int rc = prepare_ag(&b, stream, p, &costage, &small_cus)) return rc;
   const int n_counters = (int)(a->M / 128);
   const int n_flags = (int)(kSplitFlagBytes / 4);
   const int n = std::max(n_flags, n_counters);
@@ -455,7 +533,7 @@ int mk_ag_gemm_noalloc(const mk_ag_gemm_args* a, void* stream) {
                      static_cast<uint32_t*>(base), n_flags, b.stage_counters, n_counters);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "mk_ag_gemm_noalloc scratch clear");
-  return launch_ag(p, costage, stream);
+  return launch_ag(p, costage, small_cus, stream);
 }
 
 int64_t mk_ag_gemm_noalloc_scratch_bytes(void) { return kNoAllocBytes; }
@@ -548,7 +626,10 @@ int rs_launch(const mk_gemm_rs_args* a, const void* peer_reduced, uint16_t* full
     }
   }
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, fn)) return rc;
-  plan_split(p, bm, a->split_ws, a->split_ws_bytes);
+  if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
+    const int rc = small_fused(p, true, d.cus, stream, fn);
+    if (rc != kNoSmallPlan) return rc;
+  }
   hipError_t e = costage_waves ? mk::launch_gemm_costaged(p, mk::kEpiReduce, costage_waves * total,
                                                           static_cast<hipStream_t>(stream))
                                : mk::launch_gemm(p, bm, mk::kEpiReduce, static_cast<hipStream_t>(stream));
@@ -659,7 +740,10 @@ int mk_gemm_ar(const mk_gemm_ar_args* a, void* stream) {
     }
   }
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm_ar")) return rc;
-  plan_split(p, bm, a->split_ws, a->split_ws_bytes);
+  if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
+    const int rc = small_fused(p, true, d.cus, stream, "mk_gemm_ar launch");
+    if (rc != kNoSmallPlan) return rc;
+  }
   hipError_t e = costage_waves ? mk::launch_gemm_costaged(p, mk::kEpiReduce, costage_waves * total,
                                                           static_cast<hipStream_t>(stream))
                                : mk::launch_gemm(p, bm, mk::kEpiReduce, static_cast<hipStream_t>(stream));

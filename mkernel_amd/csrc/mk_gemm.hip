@@ -198,6 +198,19 @@ __device__ void coop_stage(const GemmKParams& p, int stride, int& q, int& batch,
   }
 }
 
+// Every block staged by a kernel of its own, before a GEMM that reads them
+// (the small-tile kernel: a launch of few tiles leaves most CUs idle while
+// its own workgroups copy).  One piece per workgroup and step; 256 threads of
+// 16 loads in flight copy a 64 KB piece at once.
+__global__ __launch_bounds__(256) void stage_all_kernel(GemmKParams p) {
+  for (int q = blockIdx.x; q < p.st_nblocks * kPieces; q += gridDim.x) {
+    const int b = stage_piece<256, 16>(p, q);
+    wait_vmem_all();
+    __syncthreads();
+    if (threadIdx.x == 0) count_piece(p, b);
+  }
+}
+
 // Claimed staging (st_coop 3), the compute workgroups' side: pieces are
 // handed out in stage order through the launch's claim word (st_claim[0]),
 // which the co-resident staging kernel (stage_kernel) draws from one piece
@@ -275,90 +288,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_vgpr(32))) void stage
 // Epilogue of one BM x BN tile.  acc[i][j][4a+b] is C[m][n] with
 // m = m0 + wm*WTM + 32i + ml and n (in tile) = wn*WTN + 32j + 8a + 4kg + b.
 // ---------------------------------------------------------------------------
-// Reduce epilogue of an owned tile, row-major: each 32-row block of the
-// wave's fp32 accumulators goes through the wave's LDS region (rows of WTN
-// fp32, pitch padded by 16 bytes) and comes back 8 columns per lane with
-// consecutive lanes along a row; the lane then loads the same 8 columns of
-// every peer's bf16 partial (16 bytes per peer: whole row segments per
-// instruction, 4 peers' loads in flight, the remainder as one more group),
-// adds them in rank order in fp32
-// (deterministic, one rounding) and stores 16 bytes of the owned output.
-// In the accumulator layout every load and store instruction would touch
-// 32 rows with 8 bytes each.
-template <class C>
-__device__ __forceinline__ void reduce_rows(const GemmKParams& p, f32x16 (&acc)[C::FM][C::FN], int lrow0, int col0,
-                                            char* smem, int wave, int lane) {
-  constexpr int PITCH = C::WTN * 4 + 16;  // bytes per LDS row (fp32)
-  constexpr int LPR = C::WTN / 8;         // lanes per row (8 columns each)
-  constexpr int RPI = 64 / LPR;           // rows per instruction
-  constexpr int kPeers = 4;               // peer loads in flight per lane
-  static_assert(64 % LPR == 0 && 32 % RPI == 0, "reduce_rows shape");
-  int l = lane;
-  asm volatile("" : "+v"(l));  // keep lane-derived addressing below the K loop
-  const int ml = l & 31, kg = l >> 5;
-  char* reg = smem + wave * 32 * PITCH;
-  const int rr = l / LPR, cc = l % LPR;
-  const int64_t peer_stride = (int64_t)p.rs_own_rows * p.ldc;
-  const int np = p.rs_npeers;
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i) {
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        f32x4 w;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) w[b] = acc[i][j][4 * a + b];
-        *reinterpret_cast<f32x4*>(reg + ml * PITCH + (32 * j + 8 * a + 4 * kg) * 4) = w;
-      }
-    wait_lgkm_all();
-    for (int r = 0; r < 32 / RPI; ++r) {
-      const int row = r * RPI + rr;
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(reg + row * PITCH + cc * 32);
-      const f32x4 hi = *reinterpret_cast<const f32x4*>(reg + row * PITCH + cc * 32 + 16);
-      float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      const uint16_t* src = p.rs_recv + (int64_t)(lrow0 + i * 32 + row) * p.ldc + col0 + cc * 8;
-      int q = 0;
-      for (; q + kPeers <= np; q += kPeers) {
-        uint4 v[kPeers];
-#pragma unroll
-        for (int u = 0; u < kPeers; ++u) v[u] = *reinterpret_cast<const uint4*>(src + (q + u) * peer_stride);
-#pragma unroll
-        for (int u = 0; u < kPeers; ++u) {
-          x[0] += bf16_lo(v[u].x); x[1] += bf16_hi(v[u].x);
-          x[2] += bf16_lo(v[u].y); x[3] += bf16_hi(v[u].y);
-          x[4] += bf16_lo(v[u].z); x[5] += bf16_hi(v[u].z);
-          x[6] += bf16_lo(v[u].w); x[7] += bf16_hi(v[u].w);
-        }
-      }
-      if (q < np) {
-        // the last np - q peers as one more group in flight (indices
-        // clamped to the last peer, so no branch splits the loads)
-        uint4 v[kPeers];
-#pragma unroll
-        for (int u = 0; u < kPeers; ++u)
-          v[u] = *reinterpret_cast<const uint4*>(src + (int64_t)min(q + u, np - 1) * peer_stride);
-#pragma unroll
-        for (int u = 0; u < kPeers; ++u)
-          if (q + u < np) {
-            x[0] += bf16_lo(v[u].x); x[1] += bf16_hi(v[u].x);
-            x[2] += bf16_lo(v[u].y); x[3] += bf16_hi(v[u].y);
-            x[4] += bf16_lo(v[u].z); x[5] += bf16_hi(v[u].z);
-            x[6] += bf16_lo(v[u].w); x[7] += bf16_hi(v[u].w);
-          }
-      }
-      uint4 o;
-      o.x = pack_bf16x2(x[0], x[1]); o.y = pack_bf16x2(x[2], x[3]);
-      o.z = pack_bf16x2(x[4], x[5]); o.w = pack_bf16x2(x[6], x[7]);
-      typedef uint32_t nt_u32x4 __attribute__((ext_vector_type(4)));
-      __builtin_nontemporal_store(nt_u32x4{o.x, o.y, o.z, o.w},
-                                  reinterpret_cast<nt_u32x4*>(p.rs_out + (int64_t)(lrow0 + i * 32 + row) * p.ldc +
-                                                              col0 + cc * 8));
-    }
-    wait_lgkm_all();  // this block's reads are done before the next block's writes
-  }
-}
-
 template <class C, int EPI>
 __device__ __forceinline__ void store_tile(const GemmKParams& p, f32x16 (&acc)[C::FM][C::FN], int m0, int tn,
                                            int tid, char* smem) {
@@ -1053,6 +982,12 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
   // still copies its shares of the ranges staged before that round
   if (sp.round_need && sp.gsize > 0)
     for (int w = n_full_mine; w < sp.n_rounds; ++w) alt_stage<C::NT>(p, cons_id, sp, w);
+  // The reduce epilogue's launches have no K-split tail: its partial exchange
+  // beside the fold needed 272 spilled registers, and a whole partial round,
+  // whose idle CUs leave the others a higher clock, was faster at all but one
+  // of nine shapes (16384x3584x3584 435 -> 367 us with staged partials,
+  // 10240x2048x1024 115 -> 74).
+  if constexpr (EPI == kEpiReduce) return;
   if (cons_id >= n_tail_units) return;
   // The K-split unit: tail tile full + tail_idx (unpermuted), K part `part`.
   const int tail_idx = cons_id / sk_split;
@@ -1398,6 +1333,23 @@ __global__ void epoch_advance_kernel(uint32_t* epoch_ptr) {
     if (e == 0u) e = 1u;
     __hip_atomic_store(epoch_ptr, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+hipError_t launch_stage_all(const GemmKParams& p, int grid, hipStream_t stream) {
+  hipLaunchKernelGGL(stage_all_kernel, dim3(grid), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+// Every done flag of an all-reduce whose rows an earlier launch finished.
+__global__ void publish_done_kernel(uint32_t* done, int n, const uint32_t* epoch_ptr, uint32_t epoch) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n)
+    publish_flag(done + i, epoch_ptr ? __hip_atomic_load(epoch_ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : epoch);
+}
+
+hipError_t launch_publish_done(uint32_t* done, int n, const uint32_t* epoch_ptr, uint32_t epoch, hipStream_t stream) {
+  hipLaunchKernelGGL(publish_done_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, done, n, epoch_ptr, epoch);
+  return hipGetLastError();
 }
 
 hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream) {

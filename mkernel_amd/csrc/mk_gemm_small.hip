@@ -125,7 +125,7 @@ __device__ __forceinline__ void parts_in(const float* slot0, const int* where, i
     for (int b = 0; b < 4; ++b) acc[u / (C::FN * 4)][(u / 4) % C::FN][4 * (u % 4) + b] = s[u][b];
 }
 
-template <class C>
+template <class C, bool REDUCE>
 __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -175,6 +175,10 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
     st += n;
     int tm, tn;
     decode_grouped((int)t, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
+    // The rows to fold cost more than the others and are neighbours: each
+    // eighth of the columns starts its walk over the rows another eighth
+    // further on, so that the fold falls on every XCD.
+    if (REDUCE) tm = (tm + tn * 8 / p.tiles_n * ((p.tiles_m + 7) / 8)) % p.tiles_m;
     const int m0 = __builtin_amdgcn_readfirstlane(tm * C::BM), n0 = __builtin_amdgcn_readfirstlane(tn * C::BN);
     const u32x4_t rA = make_rsrc_v(p.A + (int64_t)m0 * p.lda, (uint32_t)(C::BM * p.lda * 2));
     const u32x4_t rB = make_rsrc_v(p.B, (uint32_t)(p.K * p.ldb * 2));
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
       compute();
     }
     __syncthreads();  // the ring is free: the exchange and the store use it
-    if (n < (int)nk) {
+    if (!REDUCE && n < (int)nk) {
       // first and last workgroup with a part of this tile
       const uint32_t f0 = t * nk, f1 = f0 + nk - 1;
       const uint32_t w0 = (uint32_t)(((uint64_t)(f0 + 1) * G - 1) / total);
@@ -295,86 +299,154 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
       parts_in<C>(slot0, sh + 1, parts, own, acc, tid);
       __syncthreads();  // sh is read: the store reuses the LDS
     }
-    store_rows<C>(p.C + (int64_t)(m0 + wm * C::WTM) * p.ldc + n0 + wn * C::WTN, p.ldc, acc, smem, wave, lane);
+    if (REDUCE && m0 >= p.rs_own_row0 && m0 < p.rs_own_row0 + p.rs_own_rows) {
+      static_assert(!REDUCE || C::WAVES * 32 * (C::WTN * 4 + 16) <= C::LDS_BYTES, "fold rows in LDS");
+      reduce_rows<C, 8>(p, acc, m0 - p.rs_own_row0 + wm * C::WTM, n0 + wn * C::WTN, smem, wave, lane);
+    } else {
+      // with the fold these are the would-be sends: written once, not read here
+      store_rows<C, C::FN, REDUCE>(p.C + (int64_t)(m0 + wm * C::WTM) * p.ldc + n0 + wn * C::WTN, p.ldc, acc, smem, wave,
+                                   lane);
+    }
     if (st < end) __syncthreads();  // the ring is refilled by the next tile
   }
 }
 
-template <class C>
+template <class C, bool REDUCE>
 hipError_t launch_s(const GemmSmallParams& p, int grid, hipStream_t stream) {
   static PerDeviceFlag attr_set;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (!attr_set.is_set(dev)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_small_kernel<C>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_small_kernel<C, REDUCE>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
     if (e != hipSuccess) return e;
     attr_set.set(dev);
   }
-  hipLaunchKernelGGL((gemm_small_kernel<C>), dim3(grid), dim3(C::NT), C::LDS_BYTES, stream, p);
+  hipLaunchKernelGGL((gemm_small_kernel<C, REDUCE>), dim3(grid), dim3(C::NT), C::LDS_BYTES, stream, p);
   return hipGetLastError();
 }
 
-// The tile shapes, and what a tile costs in us: start + stages x slope, with
-// slope = base + load x (workgroups of the busiest round / CUs) while every
-// CU holds at most one (a full chip clocks lower and shares its L2s), and
-// base + load + more x (k - 1) with k > 1 of them on a CU (`per_cu` fit its
-// LDS together; more run in rounds).  `meet` is what parts of a tile cost to
-// meet.  Fitted to N(0, 1/K) operands at 23 shapes of 128 .. 4096 rows, 256 ..
-// 8192 columns and 512 .. 8192 K on one MI355X.
+// The tile shapes and what they cost, in us.  A launch of g tiles runs in
+// rounds of per_cu x CUs workgroups (what fits the LDS of a CU together), each
+//   round + stages x slope(x),   x = the round's workgroups per CU,
+// slope = one + load x while no CU holds two, else two + more (x - 1): a full
+// chip clocks lower and shares its caches.  `start` comes once, `meet` when
+// the parts of a tile have to meet.  Fitted to N(0, 1/K) operands at 40 shapes
+// of 128 .. 10240 rows, 256 .. 8192 columns and 256 .. 8192 K on one MI355X.
+// The two-stage rings (128 x 128 at 64 KB, 64 x 64 at 32 KB) hide one tile's
+// first loads and its store behind its neighbours on the CU, which is worth
+// more than a deeper ring when many short tiles follow each other:
+// 10240x6656x512 takes 82 us with them, 107 with one 128 KB ring per CU.
 struct TileCost {
   int bm, bn, per_cu;
-  double start, base, load, more, meet;
+  double start, round, one, load, two, more, meet;
 };
 constexpr TileCost kTiles[] = {
-    {64, 64, 3, 3.0, 0.235, 0.0, 0.175, 7.0},
-    {128, 64, 2, 2.3, 0.380, 0.0, 0.235, 7.0},
-    {128, 128, 1, 4.0, 0.410, 0.14, 0.0, 10.0},
-    {192, 128, 1, 5.0, 0.470, 0.33, 0.0, 10.0},
-    {128, 256, 1, 4.8, 0.520, 0.38, 0.0, 14.0},
+    {64, 64, 3, 1.8, 1.2, 0.235, 0.0, 0.33, 0.125, 7.0},
+    {128, 64, 2, 0.7, 1.6, 0.380, 0.0, 0.60, 0.02, 7.0},
+    {128, 128, 1, 3.0, 1.0, 0.410, 0.14, 0.0, 0.0, 10.0},
+    {192, 128, 1, 3.0, 2.0, 0.470, 0.33, 0.0, 0.0, 10.0},
+    {128, 256, 1, 2.5, 2.3, 0.520, 0.38, 0.0, 0.0, 14.0},
+    {128, 128, 2, 3.0, 2.0, 0.530, 0.05, 0.717, 0.245, 10.0},
+    {64, 64, 5, 0.8, 2.2, 0.300, 0.0, 0.33, 0.13, 7.0},
 };
+
+double rounds_cost(const TileCost& c, int64_t g, double stages, int cus) {
+  const int64_t full = (int64_t)c.per_cu * cus;
+  auto round = [&](int64_t n) {
+    const double x = (double)n / cus;
+    return c.round + stages * (n > cus ? c.two + c.more * (x - 1) : c.one + c.load * x);
+  };
+  return c.start + (double)(g / full) * round(full) + (g % full ? round(g % full) : 0.0);
+}
 
 }  // namespace
 
 bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int cus, bool ws, int64_t ws_tiles_bytes,
-                     int ws_words, GemmSmallPlan* plan) {
+                     int ws_words, const SmallFold& fold, GemmSmallPlan* plan) {
   // offsets from 2^31 up read as zeros, so both buffer windows end below it
   if (K * ldb * 2 >= (1LL << 31)) return false;
   const int64_t nk = (K + 63) / 64;
-  double best = 0;
+  const bool reduce = fold.peers >= 0;
   bool found = false;
   for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
     const TileCost& c = kTiles[i];
-    if (M % c.bm || N % c.bn || (int64_t)c.bm * lda * 2 >= (1LL << 31)) continue;
+    if (M % c.bm || N % c.bn || (reduce && 256 % c.bm) || (int64_t)c.bm * lda * 2 >= (1LL << 31)) continue;
     const int64_t nt = (M / c.bm) * (N / c.bn);
-    if (nt > (1 << 20) || nt * nk >= (1LL << 31)) continue;
+    if (nt * nk >= (1LL << 31)) continue;
     for (int s = 1; s <= 4; ++s) {
       const int64_t g = nt * s;
-      if (s > 1 && (!ws || g > cus || nk < 4 * s || nt + g > ws_words || g * c.bm * c.bn * 4 > ws_tiles_bytes)) break;
-      const int64_t k = (g + cus - 1) / cus;                          // workgroups on the busiest CU
-      const int64_t together = k < c.per_cu ? k : c.per_cu;
-      const double rounds = (double)k / together;
-      const double fill = k > 1 ? 1.0 : (double)g / cus;
-      const double slope = c.base + c.load * fill + c.more * (together - 1);
-      const double t = rounds * (c.start + (double)((nk + s - 1) / s) * slope) + (s > 1 ? c.meet : 0.0);
-      if (!found || t < best) {
+      if (s > 1 && (!ws || reduce || g > cus || nk < 4 * s || nt + g > ws_words ||
+                    g * c.bm * c.bn * 4 > ws_tiles_bytes))
+        break;
+      double t = rounds_cost(c, g, (double)((nk + s - 1) / s), cus) + (s > 1 ? c.meet : 0.0);
+      if (reduce) t += fold_cost(fold, (double)fold.rows / c.bm * (N / c.bn), (double)c.bm * c.bn, c.per_cu * cus);
+      if (!found || t < plan->us) {
         found = true;
-        best = t;
-        *plan = {i, c.bm, c.bn, (int)g, s};
+        *plan = {i, c.bm, c.bn, (int)g, s, t};
       }
     }
   }
   return found;
 }
 
-hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, hipStream_t stream) {
-  switch (plan.tile) {
-    case 0: return launch_s<SCfg<64, 64, 2, 2, 3>>(p, plan.grid, stream);
-    case 1: return launch_s<SCfg<128, 64, 4, 1, 3>>(p, plan.grid, stream);
-    case 2: return launch_s<SCfg<128, 128, 4, 2, 4>>(p, plan.grid, stream);
-    case 3: return launch_s<SCfg<192, 128, 2, 4, 4>>(p, plan.grid, stream);
-    case 4: return launch_s<SCfg<128, 256, 2, 4, 3>>(p, plan.grid, stream);
+namespace {
+double persistent_round(double tiles, double stages, int cus) { return 3.8 + stages * (0.24 + 0.55 * tiles / cus); }
+}  // namespace
+
+int tail_split(int64_t rest, int64_t K, int cus, double* us) {
+  const double stages = (double)K / 32;
+  int best = 1;
+  double t = persistent_round((double)rest, stages, cus);
+  for (int s = 2; s <= 4 && rest * s <= cus && K / 32 >= 4 * s; ++s) {
+    const double ts = persistent_round((double)(rest * s), stages / s, cus) + 10.0 + 1.5 * s;
+    if (ts < t) {
+      t = ts;
+      best = s;
+    }
+  }
+  if (us) *us = t;
+  return best;
+}
+
+double persistent_cost(int64_t tiles, int64_t K, int cus, bool split) {
+  const double stages = (double)K / 32;
+  double t = 5.0 + (double)(tiles / cus) * persistent_round(cus, stages, cus);
+  const int64_t rest = tiles % cus;
+  if (rest && split && tiles > cus) {
+    double tail;
+    tail_split(rest, K, cus, &tail);
+    t += tail;
+  } else if (rest) {
+    t += persistent_round((double)rest, stages, cus);
+  }
+  return t;
+}
+
+double fold_cost(const SmallFold& f, double tiles, double tile_elems, double at_once) {
+  if (f.peers <= 0) return 0.0;
+  const double chip = tiles * tile_elems * 2 * f.peers / 7e6, one = tile_elems * 2 * f.peers / 0.06e6;
+  const double own = one * (double)(int64_t)((tiles + at_once - 1) / at_once);
+  return chip > own ? chip : own;
+}
+
+hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, bool reduce, hipStream_t stream) {
+  const int grid = plan.grid;
+  switch (plan.tile * 2 + reduce) {
+    case 0: return launch_s<SCfg<64, 64, 2, 2, 3>, false>(p, grid, stream);
+    case 1: return launch_s<SCfg<64, 64, 2, 2, 3>, true>(p, grid, stream);
+    case 2: return launch_s<SCfg<128, 64, 4, 1, 3>, false>(p, grid, stream);
+    case 3: return launch_s<SCfg<128, 64, 4, 1, 3>, true>(p, grid, stream);
+    case 4: return launch_s<SCfg<128, 128, 4, 2, 4>, false>(p, grid, stream);
+    case 5: return launch_s<SCfg<128, 128, 4, 2, 4>, true>(p, grid, stream);
+    case 6: return launch_s<SCfg<192, 128, 2, 4, 4>, false>(p, grid, stream);
+    case 8: return launch_s<SCfg<128, 256, 2, 4, 3>, false>(p, grid, stream);
+    case 9: return launch_s<SCfg<128, 256, 2, 4, 3>, true>(p, grid, stream);
+    case 10: return launch_s<SCfg<128, 128, 2, 4, 2>, false>(p, grid, stream);
+    case 11: return launch_s<SCfg<128, 128, 2, 4, 2>, true>(p, grid, stream);
+    case 12: return launch_s<SCfg<64, 64, 2, 2, 2>, false>(p, grid, stream);
+    case 13: return launch_s<SCfg<64, 64, 2, 2, 2>, true>(p, grid, stream);
   }
   return hipErrorInvalidValue;
 }

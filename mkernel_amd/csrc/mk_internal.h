@@ -103,6 +103,9 @@ hipError_t launch_gemm(const GemmKParams& p, int bm, int epi, hipStream_t stream
 // staging kernel runs; both claim pieces through p.st_claim.
 hipError_t launch_gemm_costaged(const GemmKParams& p, int epi, int n_stage_waves, hipStream_t stream);
 hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream);
+// The staging of p's blocks alone (st_* fields), and the done flags alone.
+hipError_t launch_stage_all(const GemmKParams& p, int grid, hipStream_t stream);
+hipError_t launch_publish_done(uint32_t* done, int n, const uint32_t* epoch_ptr, uint32_t epoch, hipStream_t stream);
 
 // Dense GEMM of less than one round of persistent tiles (mk_gemm_small.hip).
 struct GemmSmallParams {
@@ -115,16 +118,42 @@ struct GemmSmallParams {
   int nk;            // 64-deep K stages of a tile
   uint32_t* words;   // a ticket per tile and a header per workgroup, zero between launches
   float* ws;         // an fp32 tile per workgroup
+  // reduce epilogue: rows rs_own_row0 .. + rs_own_rows are folded with the
+  // peers' staged partials into rs_out, the others are stored to C
+  int rs_own_row0, rs_own_rows, rs_npeers;
+  const uint16_t* rs_recv;
+  uint16_t* rs_out;
 };
 struct GemmSmallPlan {
   int tile, bm, bn;  // index into the kernel's tile table, and its shape
   int grid, split;   // workgroups, and parts of each tile along K
+  double us;         // estimated time
 };
+// The fold of a reduce epilogue: `rows` rows with `peers` partials each
+// (peers < 0: no such epilogue).
+struct SmallFold {
+  int peers;
+  int64_t rows;
+};
+// Estimated us of folding `tiles` tiles, `at_once` workgroups at a time: the
+// chip takes 7 TB/s of partials beside its products, one workgroup 60 GB/s.
+double fold_cost(const SmallFold& f, double tiles, double tile_elems, double at_once);
 // The tile and split with the least estimated time; false: no tile fits.
 // ws: a workspace of ws_words words and ws_tiles_bytes of tiles is there.
 bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int cus, bool ws, int64_t ws_tiles_bytes,
-                     int ws_words, GemmSmallPlan* plan);
-hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, hipStream_t stream);
+                     int ws_words, const SmallFold& fold, GemmSmallPlan* plan);
+// Parts along K (1..4) for `rest` 256 x 256 tiles of a last round on `cus`
+// workgroups, and its estimated us: splitting fills the idle CUs, which then
+// clock lower, and costs the parts' exchange, about 13 us for two of them.
+// Measured, whole against split tail: 10240x2048x1024 (64 tiles) 54 against
+// 80 us, 16384x6656x416 (128) 122 against 137, 16384x3584x3584 (128) equal,
+// 9216x2048x3584 (32) 153 against 146, 16384x3584x8192 (128) 745 against 735.
+int tail_split(int64_t rest, int64_t K, int cus, double* us);
+// Estimated us of the persistent kernel on `tiles` 256 x 256 tiles (split:
+// with a workspace for the K-split of its tail).  Fitted like the tile table:
+// 4096^3 106-118 measured, 8192x8192x512 71, 8192x3584x8192 382.
+double persistent_cost(int64_t tiles, int64_t K, int cus, bool split);
+hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, bool reduce, hipStream_t stream);
 
 struct PermuteKParams {
   const uint16_t* tokens;

@@ -1,6 +1,7 @@
 // mk_tile.h — building blocks of the tiled bf16 GEMM kernels (gfx950): HBM ->
 // LDS DMA with hand-counted completion, the transposing LDS read, the grouped
-// tile order and the row-major bf16 store of a wave's accumulators.
+// tile order, the row-major bf16 store of a wave's accumulators and the fold of
+// peers' partials into them.
 #pragma once
 #include "mk_device.h"
 
@@ -158,6 +159,89 @@ __device__ __forceinline__ void store_rows(uint16_t* base, int64_t ldc, f32x16 (
       } else {
         *dst = v;
       }
+    }
+    wait_lgkm_all();  // this block's reads are done before the next block's writes
+  }
+}
+
+// Reduce epilogue of an owned tile, row-major: each 32-row block of the
+// wave's fp32 accumulators goes through the wave's LDS region (rows of WTN
+// fp32, pitch padded by 16 bytes) and comes back 8 columns per lane with
+// consecutive lanes along a row; the lane then loads the same 8 columns of
+// every peer's bf16 partial (16 bytes per peer: whole row segments per
+// instruction, kPeers peers' loads in flight, the remainder as one more group),
+// adds them in rank order in fp32
+// (deterministic, one rounding) and stores 16 bytes of the owned output.
+// In the accumulator layout every load and store instruction would touch
+// 32 rows with 8 bytes each.
+template <class C, int kPeers = 4, class P>
+__device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::FN], int lrow0, int col0,
+                                            char* smem, int wave, int lane) {
+  constexpr int PITCH = C::WTN * 4 + 16;  // bytes per LDS row (fp32)
+  constexpr int LPR = C::WTN / 8;         // lanes per row (8 columns each)
+  constexpr int RPI = 64 / LPR;           // rows per instruction
+  static_assert(64 % LPR == 0 && 32 % RPI == 0, "reduce_rows shape");
+  int l = lane;
+  asm volatile("" : "+v"(l));  // keep lane-derived addressing below the K loop
+  const int ml = l & 31, kg = l >> 5;
+  char* reg = smem + wave * 32 * PITCH;
+  const int rr = l / LPR, cc = l % LPR;
+  const int64_t peer_stride = (int64_t)p.rs_own_rows * p.ldc;
+  const int np = p.rs_npeers;
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i) {
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        f32x4 w;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) w[b] = acc[i][j][4 * a + b];
+        *reinterpret_cast<f32x4*>(reg + ml * PITCH + (32 * j + 8 * a + 4 * kg) * 4) = w;
+      }
+    wait_lgkm_all();
+    for (int r = 0; r < 32 / RPI; ++r) {
+      const int row = r * RPI + rr;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(reg + row * PITCH + cc * 32);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(reg + row * PITCH + cc * 32 + 16);
+      float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      const uint16_t* src = p.rs_recv + (int64_t)(lrow0 + i * 32 + row) * p.ldc + col0 + cc * 8;
+      int q = 0;
+      for (; q + kPeers <= np; q += kPeers) {
+        uint4 v[kPeers];
+#pragma unroll
+        for (int u = 0; u < kPeers; ++u) v[u] = *reinterpret_cast<const uint4*>(src + (q + u) * peer_stride);
+#pragma unroll
+        for (int u = 0; u < kPeers; ++u) {
+          x[0] += bf16_lo(v[u].x); x[1] += bf16_hi(v[u].x);
+          x[2] += bf16_lo(v[u].y); x[3] += bf16_hi(v[u].y);
+          x[4] += bf16_lo(v[u].z); x[5] += bf16_hi(v[u].z);
+          x[6] += bf16_lo(v[u].w); x[7] += bf16_hi(v[u].w);
+        }
+      }
+      if (q < np) {
+        // the last np - q peers as one more group in flight (indices
+        // clamped to the last peer, so no branch splits the loads)
+        uint4 v[kPeers];
+#pragma unroll
+        for (int u = 0; u < kPeers; ++u)
+          v[u] = *reinterpret_cast<const uint4*>(src + (int64_t)min(q + u, np - 1) * peer_stride);
+#pragma unroll
+        for (int u = 0; u < kPeers; ++u)
+          if (q + u < np) {
+            x[0] += bf16_lo(v[u].x); x[1] += bf16_hi(v[u].x);
+            x[2] += bf16_lo(v[u].y); x[3] += bf16_hi(v[u].y);
+            x[4] += bf16_lo(v[u].z); x[5] += bf16_hi(v[u].z);
+            x[6] += bf16_lo(v[u].w); x[7] += bf16_hi(v[u].w);
+          }
+      }
+      uint4 o;
+      o.x = pack_bf16x2(x[0], x[1]); o.y = pack_bf16x2(x[2], x[3]);
+      o.z = pack_bf16x2(x[4], x[5]); o.w = pack_bf16x2(x[6], x[7]);
+      typedef uint32_t nt_u32x4 __attribute__((ext_vector_type(4)));
+      __builtin_nontemporal_store(nt_u32x4{o.x, o.y, o.z, o.w},
+                                  reinterpret_cast<nt_u32x4*>(p.rs_out + (int64_t)(lrow0 + i * 32 + row) * p.ldc +
+                                                              col0 + cc * 8));
     }
     wait_lgkm_all();  // this block's reads are done before the next block's writes
   }
