@@ -900,28 +900,29 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
   int total;
   if (int rc = grid_total(num_cus, d, "mk_moe_grouped_gemm", &total)) return rc;
   set_grid(p, total, 0, p.tiles_m * p.tiles_n);
-  // Few column tiles (GEMM1: 2I / 512 = 8): walk all row blocks of one
-  // weight column slice together, so an expert's row blocks share its weight
-  // fetch in one XCD's L2 (measured 15 us faster on config 5's GEMM1, and
-  // 6 us slower on GEMM2's 14 column tiles, which keeps groups of 8).
-  if (p.tiles_n <= 8) p.group_m = p.tiles_m;
-  // More column tiles without an epilogue (GEMM2: 7168 / 512 = 14): each
-  // expert's tiles together, column-major inside its run of row tiles
-  // (config-5 GEMM2 210.9 -> 203.7 us; GEMM1 + SwiGLU measured 6 us slower
-  // with it and keeps the order above).
-  if (p.tiles_n > 8 && mode == 0 && rb_expert) p.expert_order = 1;
+  // Each expert's tiles together, column-major inside its run of row tiles: an
+  // expert's activation rows are fetched once per XCD and its row tiles share
+  // each weight slice.  GEMM1 + SwiGLU against walking all row tiles of one
+  // column slice first (us, 32 experts of 7168 x 4096): 64 tokens 207 -> 200,
+  // 4096 392 -> 380, 16384 937 -> 851; GEMM2 16384 tokens 474 -> 441.
+  p.expert_order = 1;
   // The grouped GEMMs are bound by the chip's weight streaming.  When the
-  // tail round cannot be K-split (more tail tiles than half the grid),
-  // every workgroup runs the same number of whole-tile rounds either way;
-  // spreading the tiles evenly over ceil(tiles / rounds) workgroups (a
-  // multiple of 8, for the XCD remap) gives each of them more bandwidth:
-  // config-5 GEMM2 (658 tiles) 244 -> 231 us on 224 instead of 256.
+  // tail round is not K-split (more tail tiles than half the grid, or K so
+  // short that the parts' exchange costs more than it saves, see
+  // kExpertSplitK), every workgroup runs the same number of whole-tile rounds
+  // either way; spreading the tiles evenly over ceil(tiles / rounds)
+  // workgroups (a multiple of 8, for the XCD remap) gives each of them more
+  // bandwidth: config-5 GEMM2 (658 tiles) 244 -> 231 us on 224 instead of 256.
+  const bool split_k = K >= mk::kExpertSplitK;
   if (!sizes) {
-    const int ntiles = p.tiles_m * p.tiles_n, R = ntiles % p.n_cons;
-    if (num_cus <= 0 && R != 0 && 2 * R > p.n_cons) {
+    const int ntiles = p.tiles_m * p.tiles_n;
+    // few tiles with a long K: the whole grid, so that they can be split
+    if (split_k && split_ws && 2 * ntiles <= total) set_grid(p, total, 0, total);
+    const int R = ntiles % p.n_cons;
+    if (num_cus <= 0 && R != 0 && (2 * R > p.n_cons || !split_k)) {
       const int rounds = (ntiles + p.n_cons - 1) / p.n_cons;
       const int even = ((ntiles + rounds - 1) / rounds + 7) / 8 * 8;
-      if (even < p.n_cons) set_grid(p, even, 0, ntiles);
+      if (even < p.n_cons) set_grid(p, even, 0, std::max(even, ntiles));
     }
   }
   if (int rc = check_ws(split_ws, split_ws_bytes, "mk_moe_grouped_gemm")) return rc;
@@ -937,7 +938,7 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
       p.sk_flags = static_cast<uint32_t*>(split_ws);
       p.sk_ws = reinterpret_cast<float*>(static_cast<char*>(split_ws) + kSplitFlagBytes);
     }
-  } else {
+  } else if (split_k) {
     plan_split(p, 128, split_ws, split_ws_bytes, bn);
   }
   hipError_t e = mk::launch_gemm(p, 128, mode == 1 ? mk::kEpiSwiGLU : mk::kEpiStore, stream, bn);

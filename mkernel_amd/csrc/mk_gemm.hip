@@ -529,6 +529,33 @@ __device__ __forceinline__ int xcd_slot(int c, int n_cons, int count, bool sprea
   return x * base + min(x, rem) + j;
 }
 
+// Expert whose padded row range [beg, end) holds row `row`, from the padded
+// row counts per expert (the last expert if none does): 64 counts per step,
+// their running sum by shuffles (one load latency per 64 experts; a walk that
+// loaded one count after another took one per expert and tile).
+__device__ __forceinline__ int expert_of_row(const GemmKParams& p, int row, int& beg, int& end) {
+  const int ln = threadIdx.x & 63;
+  int base = 0;
+  for (int e0 = 0;; e0 += 64) {
+    const int n = e0 + ln < p.n_experts ? p.expert_rows[e0 + ln] : 0;
+    int incl = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(incl, d, 64);
+      if (ln >= d) incl += y;
+    }
+    const uint64_t above = __ballot(e0 + ln < p.n_experts && row < base + incl);
+    const bool last = e0 + 64 >= p.n_experts;
+    if (above || last) {
+      const int l = above ? __builtin_ctzll(above) : p.n_experts - 1 - e0;
+      end = base + __shfl(incl, l, 64);
+      beg = end - __shfl(n, l, 64);
+      return e0 + l;
+    }
+    base += __shfl(incl, 63, 64);
+  }
+}
+
 template <class C, int EPI>
 __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, int n_cons, char* smem,
                                              const int* row_perm, const uint16_t* full_list, StagePlan& sp) {
@@ -539,8 +566,8 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
   const int wn = wave % C::WN;
   // Row tiles and tail split from the launch parameters, or from the device
   // row count (tiles past it are not walked; the split follows the rule the
-  // host's plan uses: R = tiles % n_cons tail tiles, each split
-  // min(4, n_cons / R, K stages / 4) ways when that is at least 2).
+  // host's plan uses: from K = kExpertSplitK on, R = tiles % n_cons tail tiles,
+  // each split min(4, n_cons / R, K stages / 4) ways when that is at least 2).
   int tiles_m = p.tiles_m, sk_split = p.sk_split, sk_full = p.sk_full;
   if constexpr (C::BM == 128) {
     if (p.rows_dev) {
@@ -550,7 +577,7 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
       sk_split = 0;
       sk_full = nt;
       const int R = nt % n_cons;
-      if (p.sk_dev && R != 0) {
+      if (p.sk_dev && R != 0 && p.K >= kExpertSplitK) {
         const int s = min(min(4, n_cons / R), (p.K / 32) / 4);
         if (s >= 2) {
           sk_split = s;
@@ -610,31 +637,40 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
       // inside the run, column-major.  A one-tile expert's column tiles
       // are consecutive, so its activation rows are fetched once per XCD;
       // a multi-tile expert's row tiles still stream each weight slice
-      // together.  The host sets this only with rb_expert.
+      // together.
       const int rt = __builtin_amdgcn_readfirstlane(t / p.tiles_n);
-      const int e = __builtin_amdgcn_readfirstlane(p.rb_expert[rt]);
-      // Run bounds 64 row tiles per step: every lane loads one table entry
-      // and a ballot finds the first entry of another expert, so a long run
-      // (a hot expert) costs one load per 64 tiles, not one per tile.
-      const int ln = threadIdx.x & 63;
       int r0 = rt, r1 = rt + 1;
-      for (;;) {  // backwards: r0 = one past the last other-expert entry below rt
-        const int idx = r0 - 1 - ln;
-        const uint64_t other = __ballot(idx < 0 || p.rb_expert[max(idx, 0)] != e);
-        if (other) {
-          r0 -= __builtin_ctzll(other);  // entries r0-1 .. r0-k share e, entry r0-1-k does not
-          break;
+      if (p.rb_expert) {
+        const int e = __builtin_amdgcn_readfirstlane(p.rb_expert[rt]);
+        // Run bounds 64 row tiles per step: every lane loads one table entry
+        // and a ballot finds the first entry of another expert, so a long run
+        // (a hot expert) costs one load per 64 tiles, not one per tile.
+        const int ln = threadIdx.x & 63;
+        for (;;) {  // backwards: r0 = one past the last other-expert entry below rt
+          const int idx = r0 - 1 - ln;
+          const uint64_t other = __ballot(idx < 0 || p.rb_expert[max(idx, 0)] != e);
+          if (other) {
+            r0 -= __builtin_ctzll(other);  // entries r0-1 .. r0-k share e, entry r0-1-k does not
+            break;
+          }
+          r0 -= 64;
         }
-        r0 -= 64;
-      }
-      for (;;) {  // forwards: r1 = the first other-expert entry at or above rt + 1
-        const int idx = r1 + ln;
-        const uint64_t other = __ballot(idx >= tiles_m || p.rb_expert[min(idx, tiles_m - 1)] != e);
-        if (other) {
-          r1 += __builtin_ctzll(other);
-          break;
+        for (;;) {  // forwards: r1 = the first other-expert entry at or above rt + 1
+          const int idx = r1 + ln;
+          const uint64_t other = __ballot(idx >= tiles_m || p.rb_expert[min(idx, tiles_m - 1)] != e);
+          if (other) {
+            r1 += __builtin_ctzll(other);
+            break;
+          }
+          r1 += 64;
         }
-        r1 += 64;
+      } else {
+        // the tiles whose first row is in the expert's range (the last expert
+        // also takes the rows past every range)
+        int beg, end;
+        const int e = expert_of_row(p, rt * C::BM, beg, end);
+        r0 = (beg + C::BM - 1) / C::BM;
+        r1 = e == p.n_experts - 1 ? tiles_m : (end + C::BM - 1) / C::BM;
       }
       r0 = __builtin_amdgcn_readfirstlane(r0);
       r1 = __builtin_amdgcn_readfirstlane(r1);
@@ -657,14 +693,8 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
       const int e = __builtin_amdgcn_readfirstlane(min(max(p.rb_expert[tm], 0), p.n_experts - 1));
       Bp += (int64_t)e * p.b_expert_stride;
     } else if (p.expert_rows) {
-      // Expert whose padded row range holds row m0 (prefix walk over the
-      // per-expert padded counts; E is small).
-      int e = 0, end = 0;
-      for (; e < p.n_experts; ++e) {
-        end += p.expert_rows[e];
-        if (m0 < end) break;
-      }
-      e = __builtin_amdgcn_readfirstlane(min(e, p.n_experts - 1));
+      int beg, end;
+      const int e = __builtin_amdgcn_readfirstlane(expert_of_row(p, m0, beg, end));
       Bp += (int64_t)e * p.b_expert_stride;
     }
 
@@ -988,10 +1018,11 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
   // of nine shapes (16384x3584x3584 435 -> 367 us with staged partials,
   // 10240x2048x1024 115 -> 74).
   if constexpr (EPI == kEpiReduce) return;
-  if (cons_id >= n_tail_units) return;
+  const int unit = C::BM == 128 ? xcd_slot(cons_id, n_cons, n_tail_units, p.xcd_remap != 0) : cons_id;
+  if (unit < 0 || unit >= n_tail_units) return;
   // The K-split unit: tail tile full + tail_idx (unpermuted), K part `part`.
-  const int tail_idx = cons_id / sk_split;
-  const int part = cons_id % sk_split;
+  const int tail_idx = unit / sk_split;
+  const int part = unit % sk_split;
   const int k0 = part * nk_all / sk_split;
   const int nk = (part + 1) * nk_all / sk_split - k0;
   f32x16 acc[C::FM][C::FN];
@@ -1228,8 +1259,8 @@ __device__ __forceinline__ void gemm_main(const GemmKParams& p) {
   int cons = blockIdx.x - p.n_prod;
   int n_cons = p.n_cons;
   if constexpr (BM == 128) {
-    // Device row count with the library's grid: when the tail round cannot
-    // be K-split (more tail tiles than half the grid), every consumer runs
+    // Device row count with the library's grid: when the tail round is not
+    // K-split (more tail tiles than half the grid, or a short K), every consumer runs
     // the same number of whole-tile rounds anyway, so spread the tiles over
     // the fewest consumers (a multiple of 8) that keep that round count —
     // the host's rule for host-sized launches; the others exit here.
@@ -1237,7 +1268,7 @@ __device__ __forceinline__ void gemm_main(const GemmKParams& p) {
       const int64_t rows = *p.rows_dev;
       const int nt = (int)min<int64_t>(p.tiles_m, max<int64_t>(rows, 0) / C::BM) * p.tiles_n;
       const int R = nt % n_cons;
-      if (R != 0 && 2 * R > n_cons) {
+      if (R != 0 && (2 * R > n_cons || p.K < kExpertSplitK)) {
         const int rounds = (nt + n_cons - 1) / n_cons;
         const int even = ((nt + rounds - 1) / rounds + 7) / 8 * 8;
         if (even < n_cons) {

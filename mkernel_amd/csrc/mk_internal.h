@@ -13,6 +13,13 @@ constexpr int kMaxSplitListTiles = 4096;  // K-split with a permuted tile order:
 constexpr int kMaxRounds = 64;   // cooperative staging between rounds: at most this many rounds
 constexpr int kPieces = 16;  // cooperative staging: pieces per 128-row block
 
+// Expert GEMMs split a tail tile along K from this K on.  The parts' exchange
+// takes 20 to 30 us: a third of a tile's time at K 7168 (6 experts of 4096
+// columns, 48 tiles: 155 us whole, 92 split), more than it saves at 2048 (280
+// tiles: 134 us with the 24 of the tail split, 114 on 144 workgroups; 84
+// tiles: 40 whole, 51 split).
+constexpr int kExpertSplitK = 4096;
+
 struct GemmKParams {
   // operands
   const uint16_t* A;
