@@ -914,10 +914,11 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
   // workgroups (a multiple of 8, for the XCD remap) gives each of them more
   // bandwidth: config-5 GEMM2 (658 tiles) 244 -> 231 us on 224 instead of 256.
   const bool split_k = K >= mk::kExpertSplitK;
+  const int ntiles = p.tiles_m * p.tiles_n;
+  // few tiles with a long K: the whole grid, so that they can be split (with a
+  // device row count always, since only the device knows how many there are)
+  if (split_k && split_ws && (sizes || 2 * ntiles <= total)) set_grid(p, total, 0, total);
   if (!sizes) {
-    const int ntiles = p.tiles_m * p.tiles_n;
-    // few tiles with a long K: the whole grid, so that they can be split
-    if (split_k && split_ws && 2 * ntiles <= total) set_grid(p, total, 0, total);
     const int R = ntiles % p.n_cons;
     if (num_cus <= 0 && R != 0 && (2 * R > p.n_cons || !split_k)) {
       const int rounds = (ntiles + p.n_cons - 1) / p.n_cons;
