@@ -18,10 +18,17 @@
 //   count   per 256-entry chunk, per-expert counts            -> hist[e][chunk]
 //           per 256 tokens, routed entries                     -> tok[t]
 //   plan    one block: per-expert totals and chunk prefixes, padded expert
-//           offsets, R and R_pad, per-expert tables           -> base[e][chunk]
+//           offsets, R and R_pad, per-expert tables
 //           exclusive prefix of tok                            -> owner_offset
 //   scatter per chunk: stable rank within the chunk, row, slot -> routed rows
 //           per 256 rows < R_pad: expert of the row, padding rows, row-block tables
+// (plan leaves the chunk prefixes relative to the expert and scatter adds the
+// expert's offset: rewriting them took 19 of plan's 30 us at 16384 tokens.)
+//
+// A small batch (a decode step: at most kSmallEntries entries, kSmallThreads
+// tokens and kSmallExperts experts) is one workgroup's work and one launch
+// (build_small_kernel): each of the three launches above takes 5 to 9 us
+// there, all of it latency.
 #include <algorithm>
 
 #include "../../include/mk.h"
@@ -37,7 +44,7 @@ struct IndexKParams {
   int T, topk, e0, n_local, row_block;
   int64_t cap;       // rows the row tables hold
   int nchunks;
-  int* hist;         // [n_local][nchunks] counts, then row bases
+  int* hist;         // [n_local][nchunks] counts, then their prefixes
   int* exp_off;      // [n_local + 1] padded row offset of each expert
   int* exp_cnt;      // [n_local] routed rows of each expert
   int* tok;          // [T] routed entries per token
@@ -173,7 +180,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(IndexKParams p) {
     const int ex = block_exclusive_scan<kPlanThreads>(padded, s, tot);
     if (e < p.n_local) {
       p.exp_off[e] = carry + ex;
-      if (e < kPlanThreads) cnt_s[e] = carry + ex;  // now the expert's row offset
       if (p.out.padded_tokens_per_expert) p.out.padded_tokens_per_expert[e] = padded;
       if (p.out.local_rb_per_expert) p.out.local_rb_per_expert[e] = cnt / p.row_block;
     }
@@ -190,12 +196,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(IndexKParams p) {
     p.sizes[1] = carry;
   }
   __syncthreads();
-  // chunk prefixes become absolute row bases
-  for (int e = wave; e < p.n_local; e += kPlanThreads / 64) {
-    int* h = p.hist + (int64_t)e * p.nchunks;
-    const int off = e < kPlanThreads ? cnt_s[e] : p.exp_off[e];
-    for (int c = lane; c < p.nchunks; c += 64) h[c] += off;
-  }
   // token CSR offsets: exclusive prefix of the per-token counts (the
   // offsets pass, merged into the same launch), kPlanThreads x kTokSeg
   // tokens per block scan
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kChunk) void scatter_kernel(IndexKParams p) {
     __syncthreads();
     if (e >= 0) {
       for (int w = 0; w < wave; ++w) rank += wcnt[w * p.n_local + e];
-      const int64_t row = (int64_t)p.hist[(int64_t)e * p.nchunks + blockIdx.x] + rank;
+      const int64_t row = (int64_t)p.exp_off[e] + p.hist[(int64_t)e * p.nchunks + blockIdx.x] + rank;
       const int t = (int)(i / p.topk), k = (int)(i % p.topk);
       // slot: the token's routed entries in row order = (expert, k) order
       int before = 0;
@@ -308,6 +308,138 @@ __global__ __launch_bounds__(kChunk) void scatter_kernel(IndexKParams p) {
   }
 }
 
+constexpr int kSmallThreads = 1024, kSmallEntries = 4096, kSmallExperts = 256;
+
+// The whole build in one workgroup: entries i = round * kSmallThreads + thread,
+// their experts in LDS; per round, ranks inside each wave by one ballot per
+// distinct expert, plus the counts of earlier waves and rounds.
+__global__ __launch_bounds__(kSmallThreads) void build_small_kernel(IndexKParams p) {
+  constexpr int W = kSmallThreads / 64, kRounds = kSmallEntries / kSmallThreads;
+  __shared__ int16_t el[kSmallEntries];         // local expert of each entry, -1: not here
+  __shared__ int wcnt[W * kSmallExperts];
+  __shared__ int cnt[kSmallExperts];            // routed rows so far, at the end of each expert
+  __shared__ int off[kSmallExperts + 1];        // padded row offset of each expert
+  __shared__ int tok[kSmallThreads];            // first slot of each token
+  __shared__ int s[W + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = p.T * p.topk, E = p.n_local;
+  const mk_moe_index& o = p.out;
+  int ex[kRounds], rank[kRounds];
+  float gate[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int i = r * kSmallThreads + tid;
+    ex[r] = i < n ? local_expert(p, i) : -1;
+    gate[r] = i < n ? p.gates[i] : 0.f;
+    rank[r] = 0;
+    if (i < n) el[i] = (int16_t)ex[r];
+  }
+  if (tid < E) cnt[tid] = 0;
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    if (r * kSmallThreads >= n) break;
+    for (int x = lane; x < E; x += 64) wcnt[wave * E + x] = 0;  // the wave's own counts
+    uint64_t pending = __ballot(ex[r] >= 0);
+    while (pending) {
+      const int e = __shfl(ex[r], __builtin_ctzll(pending), 64);
+      const uint64_t m = __ballot(ex[r] == e);
+      if (ex[r] == e) rank[r] = __popcll(m & ((1ull << lane) - 1ull));
+      if (lane == 0) wcnt[wave * E + e] = __popcll(m);
+      pending &= ~m;
+    }
+    __syncthreads();
+    // counts of earlier waves, and of earlier rounds: one thread per expert
+    if (tid < E) {
+      int run = cnt[tid];
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const int c = wcnt[w * E + tid];
+        wcnt[w * E + tid] = run;
+        run += c;
+      }
+      cnt[tid] = run;
+    }
+    __syncthreads();
+    if (ex[r] >= 0) rank[r] += wcnt[wave * E + ex[r]];
+    __syncthreads();  // wcnt is refilled by the next round
+  }
+  if (n == 0) __syncthreads();
+  const int c = tid < E ? cnt[tid] : 0;
+  const int padded = (c + p.row_block - 1) / p.row_block * p.row_block;
+  int R_pad, R;
+  const int my_off = block_exclusive_scan<kSmallThreads>(padded, s, R_pad);
+  if (tid < E) {
+    off[tid] = my_off;
+    if (o.padded_tokens_per_expert) o.padded_tokens_per_expert[tid] = padded;
+    if (o.local_rb_per_expert) o.local_rb_per_expert[tid] = c / p.row_block;
+  }
+  int routed = 0;
+  if (tid < p.T)
+    for (int k = 0; k < p.topk; ++k) routed += el[tid * p.topk + k] >= 0;
+  const int slot0 = block_exclusive_scan<kSmallThreads>(routed, s, R);
+  tok[tid] = slot0;
+  if (o.owner_offset) {
+    if (tid < p.T) o.owner_offset[tid] = slot0;
+    if (tid == 0) o.owner_offset[p.T] = R;
+  }
+  if (tid == 0) {
+    off[E] = R_pad;
+    p.sizes[0] = R;
+    p.sizes[1] = R_pad;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int e = ex[r];
+    if (e < 0) continue;
+    const int i = r * kSmallThreads + tid, t = i / p.topk, k = i - t * p.topk;
+    const int64_t row = off[e] + rank[r];
+    if (row >= p.cap) continue;  // past the capacity: sizes reports R_pad > cap
+    if (o.pull_indices) {
+      o.pull_indices[3 * row + 0] = 0;
+      o.pull_indices[3 * row + 1] = 0;
+      o.pull_indices[3 * row + 2] = t;
+    }
+    if (o.row_weight) o.row_weight[row] = gate[r];
+    if (o.row_to_owner) o.row_to_owner[row] = 0;
+    if (o.owner_offset) {
+      // slot: the token's routed entries in row order = (expert, k) order
+      int slot = tok[t];
+      for (int k2 = 0; k2 < p.topk; ++k2) {
+        const int e2 = el[t * p.topk + k2];
+        slot += e2 >= 0 && (e2 < e || (e2 == e && k2 < k));
+      }
+      if (o.row_to_slot) o.row_to_slot[row] = slot;
+      if (o.slot_to_row) o.slot_to_row[slot] = (int32_t)row;
+    }
+  }
+  for (int64_t r = tid; r < R_pad && r < p.cap; r += kSmallThreads) {
+    int lo = 0, hi = E - 1;  // expert of row r: last e with off[e] <= r
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) / 2;
+      if (off[mid] <= r) lo = mid;
+      else hi = mid - 1;
+    }
+    const int64_t ie = r - off[lo];
+    if (o.row_expert) o.row_expert[r] = lo;
+    if (ie >= cnt[lo]) {
+      if (o.pull_indices) {
+        o.pull_indices[3 * r + 0] = -1;
+        o.pull_indices[3 * r + 1] = -1;
+        o.pull_indices[3 * r + 2] = -1;
+      }
+      if (o.row_weight) o.row_weight[r] = 0.f;
+      if (o.row_to_slot) o.row_to_slot[r] = 0;
+      if (o.row_to_owner) o.row_to_owner[r] = -1;
+    }
+    if (r % p.row_block == 0) {
+      if (o.rb_expert) o.rb_expert[r / p.row_block] = lo;
+      if (o.rb_rows)
+        o.rb_rows[r / p.row_block] = (int)max((int64_t)0, min((int64_t)p.row_block, (int64_t)cnt[lo] - ie));
+    }
+  }
+}
+
 int64_t index_workspace_bytes(int T, int topk, int n_local) {
   const int64_t nchunks = ((int64_t)T * topk + kChunk - 1) / kChunk;
   const int64_t ints = (int64_t)n_local * (nchunks > 0 ? nchunks : 1) + 2 * (int64_t)n_local + 1 + T;
@@ -331,6 +463,10 @@ hipError_t launch_build_indices(const int32_t* ids, const float* gates, int T, i
   p.tok = p.exp_cnt + n_local;
   p.sizes = sizes;
   p.out = out;
+  if ((int64_t)T * topk <= kSmallEntries && T <= kSmallThreads && n_local <= kSmallExperts) {
+    hipLaunchKernelGGL(build_small_kernel, dim3(1), dim3(kSmallThreads), 0, stream, p);
+    return hipGetLastError();
+  }
   // (no routed entries: plan sees nchunks = 0 and empty experts)
   const int64_t tblocks = ((int64_t)T + kChunk - 1) / kChunk;
   const int64_t g1 = std::max<int64_t>(p.nchunks, tblocks);
