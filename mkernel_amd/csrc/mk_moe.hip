@@ -6,6 +6,8 @@
 //     src/dispatch_gemm_glu_combine.cu:736-818 combine_gather_owner; the
 //     reference pre-rounds w*y to bf16 in its producer step, here the product
 //     stays fp32 because the rows are read in place on the same GPU).
+#include <algorithm>
+
 #include "mk_device.h"
 #include "mk_internal.h"
 
@@ -36,19 +38,25 @@ hipError_t launch_permute(const PermuteKParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// One workgroup per source token; each thread owns 8 contiguous columns.
+// One workgroup per source token (several, each with a share of the column
+// chunks, when the tokens alone do not fill the chip: the loop over chunks is a
+// chain of load latencies); each thread owns V contiguous columns, 16 bytes of
+// the output: 8 of bf16, 4 of fp32, so that neighbouring lanes store
+// neighbouring 16-byte pieces.
 // The token's (row, weight) pairs are loaded once per thread, before the
 // column loop (at most kMaxSlots of them; more fall back to the slot loop),
 // and all of a chunk's row loads are issued before they are summed: the
 // kernel is latency-bound, and the dependent owner -> slot -> row -> data
 // chain per column chunk made it so.  Sums stay in slot order
 // (deterministic, bit-identical to the plain loop).
+template <int V>
 __global__ __launch_bounds__(kThreads) void combine_kernel(CombineKParams p) {
-  constexpr int kMaxSlots = 8;
+  constexpr int kMaxSlots = 8, kWords = V / 2;  // 32-bit words of a row chunk
+  typedef uint32_t words __attribute__((ext_vector_type(kWords)));
   const int64_t t = blockIdx.x;
   const int s0 = p.owner_offset[t], s1 = p.owner_offset[t + 1];
   const int n = s1 - s0;
-  const int64_t vec = p.H / 8;
+  const int64_t vec = p.H / V;
   int rows[kMaxSlots];
   float wts[kMaxSlots];
   const bool few = n <= kMaxSlots;
@@ -60,23 +68,23 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(CombineKParams p) {
 #pragma unroll
   for (int k = 0; k < kMaxSlots; ++k)
     if (few && k < n) wts[k] = rows[k] >= 0 ? p.row_weight[rows[k]] : 0.f;
-  for (int64_t c = threadIdx.x; c < vec; c += kThreads) {
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    auto add = [&](float w, const uint4& v) {
-      acc[0] += w * bf16_lo(v.x);
-      acc[1] += w * bf16_hi(v.x);
-      acc[2] += w * bf16_lo(v.y);
-      acc[3] += w * bf16_hi(v.y);
-      acc[4] += w * bf16_lo(v.z);
-      acc[5] += w * bf16_hi(v.z);
-      acc[6] += w * bf16_lo(v.w);
-      acc[7] += w * bf16_hi(v.w);
+  for (int64_t c = (int64_t)blockIdx.y * kThreads + threadIdx.x; c < vec; c += (int64_t)gridDim.y * kThreads) {
+    float acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+    auto add = [&](float w, const words& v) {
+#pragma unroll
+      for (int i = 0; i < kWords; ++i) {
+        acc[2 * i] += w * bf16_lo(v[i]);
+        acc[2 * i + 1] += w * bf16_hi(v[i]);
+      }
     };
+    auto load = [&](int64_t row) { return *reinterpret_cast<const words*>(p.y_expert + row * p.H + c * V); };
     if (few) {
-      uint4 v[kMaxSlots];
+      words v[kMaxSlots];
 #pragma unroll
       for (int k = 0; k < kMaxSlots; ++k)
-        if (k < n && rows[k] >= 0) v[k] = *reinterpret_cast<const uint4*>(p.y_expert + (int64_t)rows[k] * p.H + c * 8);
+        if (k < n && rows[k] >= 0) v[k] = load(rows[k]);
 #pragma unroll
       for (int k = 0; k < kMaxSlots; ++k)
         if (k < n && rows[k] >= 0) add(wts[k], v[k]);
@@ -84,30 +92,33 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(CombineKParams p) {
       for (int s = s0; s < s1; ++s) {
         const int row = p.slot_to_row[s];
         if (row < 0) continue;
-        add(p.row_weight[row], *reinterpret_cast<const uint4*>(p.y_expert + (int64_t)row * p.H + c * 8));
+        add(p.row_weight[row], load(row));
       }
     }
     // the layer's output is not read again here: nontemporal stores
     // (config 5 layer -7 us against plain stores)
-    if (p.out_dtype == 0) {
-      float4* o = reinterpret_cast<float4*>(static_cast<float*>(p.y_out) + t * p.H + c * 8);
-      __builtin_nontemporal_store(f32x4{acc[0], acc[1], acc[2], acc[3]}, reinterpret_cast<f32x4*>(o));
-      __builtin_nontemporal_store(f32x4{acc[4], acc[5], acc[6], acc[7]}, reinterpret_cast<f32x4*>(o) + 1);
+    if constexpr (V == 4) {
+      __builtin_nontemporal_store(f32x4{acc[0], acc[1], acc[2], acc[3]},
+                                  reinterpret_cast<f32x4*>(static_cast<float*>(p.y_out) + t * p.H + c * V));
     } else {
-      uint4 w;
-      w.x = pack_bf16x2(acc[0], acc[1]);
-      w.y = pack_bf16x2(acc[2], acc[3]);
-      w.z = pack_bf16x2(acc[4], acc[5]);
-      w.w = pack_bf16x2(acc[6], acc[7]);
       typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-      __builtin_nontemporal_store(u4{w.x, w.y, w.z, w.w}, reinterpret_cast<u4*>(static_cast<uint16_t*>(p.y_out) + t * p.H + c * 8));
+      __builtin_nontemporal_store(u4{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]),
+                                     pack_bf16x2(acc[4], acc[5]), pack_bf16x2(acc[6], acc[7])},
+                                  reinterpret_cast<u4*>(static_cast<uint16_t*>(p.y_out) + t * p.H + c * V));
     }
   }
 }
 
 hipError_t launch_combine(const CombineKParams& p, hipStream_t stream) {
   if (p.num_tokens == 0) return hipSuccess;
-  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)p.num_tokens), dim3(kThreads), 0, stream, p);
+  const int64_t v = p.out_dtype == 0 ? 4 : 8;
+  const int64_t chunks = (p.H / v + kThreads - 1) / kThreads;
+  // workgroups per token: enough for 1024 in all, at most one per column chunk
+  const unsigned split = (unsigned)std::max<int64_t>(1, std::min<int64_t>(chunks, 1024 / p.num_tokens));
+  if (v == 4)
+    hipLaunchKernelGGL(combine_kernel<4>, dim3((unsigned)p.num_tokens, split), dim3(kThreads), 0, stream, p);
+  else
+    hipLaunchKernelGGL(combine_kernel<8>, dim3((unsigned)p.num_tokens, split), dim3(kThreads), 0, stream, p);
   return hipGetLastError();
 }
 
