@@ -16,12 +16,18 @@ from .capi import (AgGemmArgs, GemmAr2Args, GemmArArgs, GemmArgs, GemmRsArgs, Mo
                    MoeIndex, MoeIndexDevArgs, MoePermuteArgs)
 
 
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
+def _ptr(t: torch.Tensor | None) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+_raw_stream = torch._C._cuda_getCurrentRawStream  # current_stream(i).cuda_stream without the Stream object
+_device_index = torch._C._cuda_getDevice
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device_index())
 
 
 def _bf16(t: torch.Tensor, name: str) -> None:
@@ -51,9 +57,7 @@ def split_workspace(device=None, stream=None) -> torch.Tensor:
     created later with a recycled handle reuses that entry, which is safe
     because each launch leaves the workspace zeroed."""
     dev = torch.device("cuda", torch.cuda.current_device() if device is None else torch.device(device).index or 0)
-    if stream is None:
-        stream = torch.cuda.current_stream(dev)
-    key = (dev, stream.cuda_stream)
+    key = (dev, (torch.cuda.current_stream(dev) if stream is None else stream).cuda_stream)
     ws = _split_ws.get(key)
     if ws is None:
         n = int(capi.lib().mk_query_workspace_bytes(0, 0, 0, 0))
@@ -77,8 +81,14 @@ def _ws(split_ws, device) -> tuple:
     device's current stream, an explicit tensor, or none at all when
     split_ws is False."""
     if split_ws is False:
-        return None, 0
-    ws = split_workspace(device) if split_ws is None or split_ws is True else split_ws
+        return 0, 0
+    if split_ws is None or split_ws is True:
+        i = device.index
+        ws = _split_ws.get((device, _raw_stream(i))) if i is not None and device.type == "cuda" else None
+        if ws is None:
+            ws = split_workspace(device)
+    else:
+        ws = split_ws
     return ws.data_ptr(), ws.numel() * ws.element_size()
 
 
@@ -92,8 +102,8 @@ def gemm(A: torch.Tensor, B: torch.Tensor, out: torch.Tensor | None = None, num_
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
     _bf16(out, "C")
-    capi.call("mk_gemm", GemmArgs(_ptr(A), _ptr(B), _ptr(out), M, N, K, K, N, N, num_cus, tile_m, waves,
-                                  *_ws(split_ws, A.device)), _stream())
+    capi.call_values("mk_gemm", GemmArgs, _stream(), A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, K, N, N,
+                     num_cus, tile_m, waves, *_ws(split_ws, A.device))
     return out
 
 
@@ -113,10 +123,10 @@ def ag_gemm(A_shards, A_full, B, C_out, flags, stage_order, epoch: int, gated: b
     _bf16(A_full, "A_full"); _bf16(B, "B"); _bf16(C_out, "C")
     M, K = A_full.shape
     N = B.shape[1]
-    args = AgGemmArgs(_ptr(A_shards), _ptr(A_full), _ptr(B), _ptr(C_out), M, N, K, _ptr(flags), _ptr(stage_order),
-                      epoch, int(gated), num_producers, num_cus, spin_limit, _ptr(error_word), _ptr(stage_counters),
-                      *_ws(split_ws, A_full.device), _ptr(epoch_ptr), n_present)
-    capi.call("mk_ag_gemm", args, _stream())
+    capi.call_values("mk_ag_gemm", AgGemmArgs, _stream(), _ptr(A_shards), _ptr(A_full), _ptr(B), _ptr(C_out), M, N, K,
+                     _ptr(flags), _ptr(stage_order), epoch, int(gated), num_producers, num_cus, spin_limit,
+                     _ptr(error_word), _ptr(stage_counters), *_ws(split_ws, A_full.device),
+                     _ptr(epoch_ptr), n_present)
     return C_out
 
 
@@ -128,10 +138,10 @@ def gemm_rs(A, B, workspace, output, peer_src, peer_recv, world: int, rank: int,
     _bf16(A, "A"); _bf16(B, "B")
     M, K = A.shape
     N = B.shape[1]
-    args = GemmRsArgs(_ptr(A), _ptr(B), _ptr(workspace), _ptr(output), _ptr(peer_src), _ptr(peer_recv), M, N, K,
-                      world, rank, _ptr(flags), _ptr(stage_order), epoch, int(gated), num_producers, num_cus,
-                      spin_limit, _ptr(error_word), _ptr(stage_counters), *_ws(split_ws, A.device), _ptr(epoch_ptr))
-    capi.call("mk_gemm_rs", args, _stream())
+    capi.call_values("mk_gemm_rs", GemmRsArgs, _stream(), _ptr(A), _ptr(B), _ptr(workspace), _ptr(output),
+                     _ptr(peer_src), _ptr(peer_recv), M, N, K, world, rank, _ptr(flags), _ptr(stage_order), epoch,
+                     int(gated), num_producers, num_cus, spin_limit, _ptr(error_word), _ptr(stage_counters),
+                     *_ws(split_ws, A.device), _ptr(epoch_ptr))
     return output
 
 
@@ -143,10 +153,10 @@ def gemm_ar(A, B, C_final, peer_src, peer_recv, world: int, flags, stage_order, 
     _bf16(A, "A"); _bf16(B, "B"); _bf16(C_final, "C_final")
     M, K = A.shape
     N = B.shape[1]
-    args = GemmArArgs(_ptr(A), _ptr(B), _ptr(C_final), _ptr(peer_src), _ptr(peer_recv), M, N, K, world, _ptr(flags),
-                      _ptr(stage_order), epoch, int(gated), num_producers, num_cus, spin_limit, _ptr(error_word),
-                      _ptr(stage_counters), _ptr(done_flags), *_ws(split_ws, A.device), _ptr(epoch_ptr))
-    capi.call("mk_gemm_ar", args, _stream())
+    capi.call_values("mk_gemm_ar", GemmArArgs, _stream(), _ptr(A), _ptr(B), _ptr(C_final), _ptr(peer_src),
+                     _ptr(peer_recv), M, N, K, world, _ptr(flags), _ptr(stage_order), epoch, int(gated), num_producers,
+                     num_cus, spin_limit, _ptr(error_word), _ptr(stage_counters), _ptr(done_flags),
+                     *_ws(split_ws, A.device), _ptr(epoch_ptr))
     return C_final
 
 
@@ -164,11 +174,10 @@ def gemm_ar_two_shot(A, B, C_final, sends, peer_src, peer_recv, peer_reduced, wo
     _bf16(A, "A"); _bf16(B, "B"); _bf16(C_final, "C_final"); _bf16(sends, "sends")
     M, K = A.shape
     N = B.shape[1]
-    args = GemmAr2Args(_ptr(A), _ptr(B), _ptr(C_final), _ptr(sends), _ptr(peer_src), _ptr(peer_recv),
-                       _ptr(peer_reduced), M, N, K, world, rank, _ptr(flags), _ptr(stage_order), epoch, int(gated),
-                       num_producers, num_cus, spin_limit, _ptr(error_word), _ptr(stage_counters), _ptr(done_flags),
-                       *_ws(split_ws, A.device), _ptr(epoch_ptr))
-    capi.call("mk_gemm_ar_two_shot", args, _stream())
+    capi.call_values("mk_gemm_ar_two_shot", GemmAr2Args, _stream(), _ptr(A), _ptr(B), _ptr(C_final), _ptr(sends),
+                     _ptr(peer_src), _ptr(peer_recv), _ptr(peer_reduced), M, N, K, world, rank, _ptr(flags),
+                     _ptr(stage_order), epoch, int(gated), num_producers, num_cus, spin_limit, _ptr(error_word),
+                     _ptr(stage_counters), _ptr(done_flags), *_ws(split_ws, A.device), _ptr(epoch_ptr))
     return C_final
 
 
@@ -251,7 +260,7 @@ def moe_build_indices_dev(topk_ids: torch.Tensor, gates: torch.Tensor, e0: int, 
     L = capi.lib()
     wsb = int(L.mk_moe_index_workspace_bytes(T, k, n_local))
     ws = torch.empty(max(wsb, 4), dtype=torch.uint8, device=dev)
-    sizes = torch.zeros(2, dtype=torch.int64, device=dev)
+    sizes = torch.empty(2, dtype=torch.int64, device=dev)  # both words are written by the build
     idx = MoeIndex(*[_ptr(t[f]) for f, _ in MoeIndex._fields_])
     args = MoeIndexDevArgs(_ptr(ids), _ptr(g), T, k, e0, n_local, row_block, cap, _ptr(ws), wsb, _ptr(sizes), idx)
     capi.call("mk_moe_build_indices_dev", args, _stream())
@@ -274,8 +283,8 @@ def moe_permute(tokens, pull, post, tokens_per_src: int | None = None, devs_per_
     _bf16(tokens, "tokens"); _bf16(post, "post_tokens")
     R_pad, H = post.shape
     tps = tokens.shape[0] if tokens_per_src is None else tokens_per_src
-    capi.call("mk_moe_permute", MoePermuteArgs(_ptr(tokens), _ptr(pull), _ptr(post), R_pad, H, tokens.shape[0], tps,
-                                                devs_per_node, _ptr(sizes)), _stream())
+    capi.call_values("mk_moe_permute", MoePermuteArgs, _stream(), _ptr(tokens), _ptr(pull), _ptr(post), R_pad, H,
+                     tokens.shape[0], tps, devs_per_node, _ptr(sizes))
     return post
 
 
@@ -292,10 +301,9 @@ def moe_grouped_gemm(A, W, out, rb_expert=None, padded_tokens_per_expert=None, m
     K = A.shape[1]
     E, _, Nw = W.shape
     tps = A.shape[0] if tokens_per_src is None else tokens_per_src
-    args = MoeGroupedGemmArgs(_ptr(A), _ptr(W), _ptr(out), _ptr(rb_expert), _ptr(padded_tokens_per_expert),
-                              _ptr(rb_rows), R_pad, K, Nw, E, mode, num_cus, *_ws(split_ws, A.device),
-                              _ptr(gather_pull), A.shape[0], tps, devs_per_node, tile_n, _ptr(sizes))
-    capi.call("mk_moe_grouped_gemm", args, _stream())
+    capi.call_values("mk_moe_grouped_gemm", MoeGroupedGemmArgs, _stream(), _ptr(A), _ptr(W), _ptr(out),
+                     _ptr(rb_expert), _ptr(padded_tokens_per_expert), _ptr(rb_rows), R_pad, K, Nw, E, mode, num_cus,
+                     *_ws(split_ws, A.device), _ptr(gather_pull), A.shape[0], tps, devs_per_node, tile_n, _ptr(sizes))
     return out
 
 
@@ -322,8 +330,8 @@ def moe_combine(y_expert, row_weight, owner_offset, slot_to_row, y_out):
     od = 0 if y_out.dtype == torch.float32 else 1
     if od == 1 and y_out.dtype != torch.bfloat16:
         raise ValueError("y_out must be float32 or bfloat16")
-    capi.call("mk_moe_combine", MoeCombineArgs(_ptr(y_expert), _ptr(row_weight), _ptr(owner_offset), _ptr(slot_to_row),
-                                                _ptr(y_out), T, H, od), _stream())
+    capi.call_values("mk_moe_combine", MoeCombineArgs, _stream(), _ptr(y_expert), _ptr(row_weight), _ptr(owner_offset),
+                     _ptr(slot_to_row), _ptr(y_out), T, H, od)
     return y_out
 
 
@@ -342,12 +350,11 @@ def moe_ffn_combine(tokens, pull, row_weight, owner_offset, slot_to_row, w1, w2,
     R_pad = pull.shape[0]
     od = 0 if y_out.dtype == torch.float32 else 1
     tps = tokens.shape[0] if tokens_per_src is None else tokens_per_src
-    args = MoeFfnArgs(_ptr(tokens), _ptr(pull), _ptr(rb_expert), _ptr(padded_tokens_per_expert), _ptr(rb_rows),
-                      _ptr(row_weight),
-                      _ptr(owner_offset), _ptr(slot_to_row), _ptr(w1), _ptr(w2), _ptr(post), _ptr(act), _ptr(y_expert),
-                      _ptr(y_out), T, tokens.shape[0], R_pad, H, I2 // 2, E, tps, devs_per_node, od, num_cus,
-                      *_ws(split_ws, tokens.device), int(fuse_dispatch), tile_n, _ptr(sizes))
-    capi.call("mk_moe_ffn_combine", args, _stream())
+    capi.call_values("mk_moe_ffn_combine", MoeFfnArgs, _stream(), _ptr(tokens), _ptr(pull), _ptr(rb_expert),
+                     _ptr(padded_tokens_per_expert), _ptr(rb_rows), _ptr(row_weight), _ptr(owner_offset),
+                     _ptr(slot_to_row), _ptr(w1), _ptr(w2), _ptr(post), _ptr(act), _ptr(y_expert), _ptr(y_out), T,
+                     tokens.shape[0], R_pad, H, I2 // 2, E, tps, devs_per_node, od, num_cus,
+                     *_ws(split_ws, tokens.device), int(fuse_dispatch), tile_n, _ptr(sizes))
     return y_out
 
 
