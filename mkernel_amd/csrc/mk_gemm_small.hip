@@ -133,9 +133,10 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
   const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   // workgroups are dealt round-robin to the 8 XCDs: give each XCD a
-  // contiguous run of ids, hence neighbouring tiles, for its L2
-  const uint32_t G = gridDim.x;
-  const uint32_t id = (G & 7) ? blockIdx.x : (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+  // contiguous run of ids, hence neighbouring tiles, for its L2 (any G: XCD x
+  // has one id more than G / 8 while x < G % 8)
+  const uint32_t G = gridDim.x, xcd = blockIdx.x & 7;
+  const uint32_t id = xcd * (G >> 3) + min(xcd, G & 7) + (blockIdx.x >> 3);
   const uint32_t nk = p.nk, total = p.tiles_m * p.tiles_n * nk;
 
   const int ml = lane & 31, g = lane >> 5;
@@ -347,10 +348,15 @@ constexpr TileCost kTiles[] = {
     {128, 64, 2, 0.7, 1.6, 0.380, 0.0, 0.60, 0.02, 7.0},
     {128, 128, 1, 3.0, 1.0, 0.410, 0.14, 0.0, 0.0, 10.0},
     {192, 128, 1, 3.0, 2.0, 0.470, 0.33, 0.0, 0.0, 10.0},
-    {128, 256, 1, 2.5, 2.3, 0.520, 0.38, 0.0, 0.0, 14.0},
+    {128, 256, 1, 2.5, 2.3, 0.620, 0.28, 0.0, 0.0, 14.0},
     {128, 128, 2, 3.0, 2.0, 0.530, 0.05, 0.717, 0.245, 10.0},
-    {64, 64, 5, 0.8, 2.2, 0.300, 0.0, 0.33, 0.13, 7.0},
+    {64, 64, 5, 0.8, 2.2, 0.300, 0.0, 0.31, 0.155, 7.0},
 };
+// The 32 KB ring of the last: its many workgroups hide a fold's loads
+// (ReduceScatter 4096x4096x256, world 16: 27 us against 32), but a plain
+// product of tall tiles thrashes L2 with them (5504x768x896 18.5 us, 14.5 with
+// the 128 x 128 tiles at 64 KB).
+constexpr int kFoldOnly = 5;
 
 double rounds_cost(const TileCost& c, int64_t g, double stages, int cus) {
   const int64_t full = (int64_t)c.per_cu * cus;
@@ -372,6 +378,7 @@ bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, 
   bool found = false;
   for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
     const TileCost& c = kTiles[i];
+    if (c.per_cu == kFoldOnly && !reduce) continue;
     if (M % c.bm || N % c.bn || (reduce && 256 % c.bm) || (int64_t)c.bm * lda * 2 >= (1LL << 31)) continue;
     const int64_t nt = (M / c.bm) * (N / c.bn);
     if (nt * nk >= (1LL << 31)) continue;
@@ -445,7 +452,6 @@ hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan
     case 9: return launch_s<SCfg<128, 256, 2, 4, 3>, true>(p, grid, stream);
     case 10: return launch_s<SCfg<128, 128, 2, 4, 2>, false>(p, grid, stream);
     case 11: return launch_s<SCfg<128, 128, 2, 4, 2>, true>(p, grid, stream);
-    case 12: return launch_s<SCfg<64, 64, 2, 2, 2>, false>(p, grid, stream);
     case 13: return launch_s<SCfg<64, 64, 2, 2, 2>, true>(p, grid, stream);
   }
   return hipErrorInvalidValue;
