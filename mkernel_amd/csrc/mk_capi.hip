@@ -884,8 +884,12 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
   p.b_expert_stride = K * Nw;
   p.M = (int)R_pad; p.N = (int)Nw; p.K = (int)K;
   // 128 x 512 tiles stream each expert's activation rows half as often per
-  // weight byte as 128 x 256 tiles.
-  const int bn = tile_n ? tile_n : (Nw % 512 == 0 ? 512 : 256);
+  // weight byte as 128 x 256 tiles.  A handful of row blocks with a long K
+  // (at most 10, or with a device row count a capacity of fewer than 256 routed
+  // rows) makes too few of them to stream at the chip's rate: us at 512 / 256
+  // columns, K 7168, 2 blocks 56 / 43, 6 90 / 75, 9 120 / 116, 13 143 / 148.
+  const bool few = K >= mk::kExpertSplitK && (sizes ? R_pad - 127LL * E < 256 : R_pad / 128 <= 10);
+  const int bn = tile_n ? tile_n : (Nw % 512 == 0 && !few ? 512 : 256);
   p.tiles_m = (int)(R_pad / 128);
   p.tiles_n = (int)(Nw / bn);
   p.rb_expert = rb_expert;
