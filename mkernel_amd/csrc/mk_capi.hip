@@ -119,14 +119,14 @@ int64_t split_ws_bytes(int cus) { return kSplitFlagBytes + (int64_t)cus * kSplit
 // weights; as tail_split finds best for dense 256-row tiles.  The workspace holds the flag
 // words at a fixed offset (so every plan finds them zeroed) followed by
 // R*(s-1) < n_cons <= CUs partial tiles, which split_ws_bytes covers.
-void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn = 256) {
+void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn = 256, bool reduce = false) {
   const int ntiles = p.tiles_m * p.tiles_n;
   const int R = ntiles % p.n_cons;
   if (!ws || R == 0 || p.waves != 8) return;
   if (p.perm_mode != mk::kPermNone && ntiles > mk::kMaxSplitListTiles) return;
   int s = std::min(4, p.n_cons / R);
   s = std::min(s, (p.K / 32) / 4);  // keep every part at >= 4 K stages
-  if (bm == 256) s = mk::tail_split(R, p.K, p.n_cons, nullptr);
+  if (bm == 256) s = mk::tail_split(R, p.K, p.n_cons, reduce, nullptr);
   if (s < 2) return;
   const int64_t parts = (int64_t)R * (s - 1);
   if (parts * 4 > kClaimOffset || kSplitFlagBytes + parts * bm * bn * 4 > ws_bytes) return;
@@ -626,6 +626,7 @@ int rs_launch(const mk_gemm_rs_args* a, const void* peer_reduced, uint16_t* full
     }
   }
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, fn)) return rc;
+  plan_split(p, bm, a->split_ws, a->split_ws_bytes, 256, true);
   if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
     const int rc = small_fused(p, true, d.cus, stream, fn);
     if (rc != kNoSmallPlan) return rc;
@@ -740,6 +741,7 @@ int mk_gemm_ar(const mk_gemm_ar_args* a, void* stream) {
     }
   }
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm_ar")) return rc;
+  plan_split(p, bm, a->split_ws, a->split_ws_bytes, 256, true);
   if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
     const int rc = small_fused(p, true, d.cus, stream, "mk_gemm_ar launch");
     if (rc != kNoSmallPlan) return rc;

@@ -559,6 +559,10 @@ __device__ __forceinline__ int expert_of_row(const GemmKParams& p, int row, int&
 template <class C, int EPI>
 __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, int n_cons, char* smem,
                                              const int* row_perm, const uint16_t* full_list, StagePlan& sp) {
+  // Only the 128-row kernels run expert GEMMs: the expert tables and the row
+  // gather compiled into the 256-row kernels cost their K loop registers
+  // (ReduceScatter 16384x8192x3584 865 us with them).
+  constexpr bool kExpert = C::BM == 128;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -630,7 +634,7 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
   auto tile_body = [&](int t, bool permuted, int k0, int nk, f32x16 (&acc)[C::FM][C::FN], int& m0_out,
                        int& tn_out) __attribute__((always_inline)) {
     int tm, tn;
-    if (C::BM == 128 && p.expert_order) {
+    if (kExpert && p.expert_order) {
       // Expert order: tile t lies in the run of row tiles [r0, r1) that
       // share row tile t / tiles_n's expert (tiles t of that run are
       // r0 * tiles_n .. r1 * tiles_n - 1, whatever the order inside it);
@@ -687,12 +691,12 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
     const int m0 = tm * C::BM;
 
     const uint16_t* Bp = p.B;
-    if (p.rb_expert) {
+    if (kExpert && p.rb_expert) {
       // clamped like the expert_rows walk: a stale table entry must not
       // form a B base outside the weight tensor
       const int e = __builtin_amdgcn_readfirstlane(min(max(p.rb_expert[tm], 0), p.n_experts - 1));
       Bp += (int64_t)e * p.b_expert_stride;
-    } else if (p.expert_rows) {
+    } else if (kExpert && p.expert_rows) {
       int beg, end;
       const int e = __builtin_amdgcn_readfirstlane(expert_of_row(p, m0, beg, end));
       Bp += (int64_t)e * p.b_expert_stride;
@@ -702,8 +706,8 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
     // MFMAs of its 32-row blocks that hold padding only (their outputs stay
     // zero, as they would be from the zero-filled padding rows).
     int fm_active = C::FM;
-    const int rb_real = (C::BM == 128 && p.rb_rows) ? __builtin_amdgcn_readfirstlane(p.rb_rows[tm]) : C::BM;
-    if (p.rb_rows) {
+    const int rb_real = (kExpert && p.rb_rows) ? __builtin_amdgcn_readfirstlane(p.rb_rows[tm]) : C::BM;
+    if (kExpert && p.rb_rows) {
       const int real = __builtin_amdgcn_readfirstlane(p.rb_rows[tm]) - wm * C::WTM;
       fm_active = __builtin_amdgcn_readfirstlane(min(max((real + 31) / 32, 0), C::FM));
     }
@@ -724,7 +728,7 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
     // token row (src_node * devs + src_dev) * tokens_per_src + src_token;
     // padding rows (src < 0) get an offset past the buffer's end, which the
     // buffer load returns as zeros.
-    const u32x4_t rA = p.gather_pull
+    const u32x4_t rA = kExpert && p.gather_pull
                            ? make_rsrc_v(p.A, (uint32_t)(p.gather_rows * p.lda * 2))
                            : make_rsrc_v(p.A + (int64_t)m0 * p.lda, (uint32_t)(C::BM * p.lda * 2));
     const u32x4_t rB = make_rsrc_v(Bp, (uint32_t)(p.K * p.ldb * 2));
@@ -737,10 +741,10 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
     for (int i = 0; i < C::A_INST; ++i) {
       const int row = (wave * C::A_INST + i) * 16 + (lane >> 2);
       const int c = (lane & 3) ^ ((row >> 2) & 3);
-      if (C::BM == 128 && p.rb_rows && row >= rb_real) {
+      if (kExpert && p.rb_rows && row >= rb_real) {
         // padding row of an expert block: read as zeros, no memory traffic
         a_src[i] = 0x80000000u;
-      } else if (p.gather_pull) {
+      } else if (kExpert && p.gather_pull) {
         const int* pr = p.gather_pull + 3 * (int64_t)(m0 + row);
         const int64_t srow = ((int64_t)pr[0] * p.gather_devs + pr[1]) * p.gather_tps + pr[2];
         a_src[i] = (pr[0] < 0 || pr[2] < 0) ? 0x80000000u : (uint32_t)(srow * p.lda * 2 + c * 16);
@@ -1012,12 +1016,6 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
   // still copies its shares of the ranges staged before that round
   if (sp.round_need && sp.gsize > 0)
     for (int w = n_full_mine; w < sp.n_rounds; ++w) alt_stage<C::NT>(p, cons_id, sp, w);
-  // The reduce epilogue's launches have no K-split tail: its partial exchange
-  // beside the fold needed 272 spilled registers, and a whole partial round,
-  // whose idle CUs leave the others a higher clock, was faster at all but one
-  // of nine shapes (16384x3584x3584 435 -> 367 us with staged partials,
-  // 10240x2048x1024 115 -> 74).
-  if constexpr (EPI == kEpiReduce) return;
   const int unit = C::BM == 128 ? xcd_slot(cons_id, n_cons, n_tail_units, p.xcd_remap != 0) : cons_id;
   if (unit < 0 || unit >= n_tail_units) return;
   // The K-split unit: tail tile full + tail_idx (unpermuted), K part `part`.

@@ -402,12 +402,12 @@ namespace {
 double persistent_round(double tiles, double stages, int cus) { return 3.8 + stages * (0.24 + 0.55 * tiles / cus); }
 }  // namespace
 
-int tail_split(int64_t rest, int64_t K, int cus, double* us) {
+int tail_split(int64_t rest, int64_t K, int cus, bool reduce, double* us) {
   const double stages = (double)K / 32;
   int best = 1;
   double t = persistent_round((double)rest, stages, cus);
   for (int s = 2; s <= 4 && rest * s <= cus && K / 32 >= 4 * s; ++s) {
-    const double ts = persistent_round((double)(rest * s), stages / s, cus) + 10.0 + 1.5 * s;
+    const double ts = persistent_round((double)(rest * s), stages / s, cus) + (reduce ? 80.0 : 10.0 + 1.5 * s);
     if (ts < t) {
       t = ts;
       best = s;
@@ -423,7 +423,7 @@ double persistent_cost(int64_t tiles, int64_t K, int cus, bool split) {
   const int64_t rest = tiles % cus;
   if (rest && split && tiles > cus) {
     double tail;
-    tail_split(rest, K, cus, &tail);
+    tail_split(rest, K, cus, false, &tail);
     t += tail;
   } else if (rest) {
     t += persistent_round((double)rest, stages, cus);

@@ -155,7 +155,11 @@ bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, 
 // Measured, whole against split tail: 10240x2048x1024 (64 tiles) 54 against
 // 80 us, 16384x6656x416 (128) 122 against 137, 16384x3584x3584 (128) equal,
 // 9216x2048x3584 (32) 153 against 146, 16384x3584x8192 (128) 745 against 735.
-int tail_split(int64_t rest, int64_t K, int cus, double* us);
+// With the reduce epilogue the exchange costs 35 to 90 us (its registers spill
+// beside the fold: 16384x3584x3584, 128 tiles, 406 whole and 480 split with the
+// partials staged in the launch; 10240x2048x1024, 64 tiles, 84 and 127), so
+// only a K of about 14000 and more is split there.
+int tail_split(int64_t rest, int64_t K, int cus, bool reduce, double* us);
 // Estimated us of the persistent kernel on `tiles` 256 x 256 tiles (split:
 // with a workspace for the K-split of its tail).  Fitted like the tile table:
 // 4096^3 106-118 measured, 8192x8192x512 71, 8192x3584x8192 382.
