@@ -169,6 +169,12 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
     return kNoSmallPlan;
   const int64_t t256 = a->M % 256 ? 0 : (a->M / 256) * (a->N / 256);
   if (2 * t256 > cus && mk::persistent_cost(t256, a->K, cus, a->split_ws != nullptr) <= plan.us) return kNoSmallPlan;
+  // An odd number of 128-row blocks, a little over one round of 128 x 256 tiles
+  // and a long K: the persistent kernel splits the few tiles of the second
+  // round four ways (4224x2048x5504, 264 tiles: 119 us, 123 in two rounds of
+  // small tiles; at K 3072, 261 tiles: 77 and 75).
+  const int64_t t128 = (a->M / 128) * (a->N / 256);
+  if (a->M % 256 && a->split_ws && a->K >= 4096 && t128 > cus && 4 * t128 <= 5 * cus) return kNoSmallPlan;
   mk::GemmSmallParams p = small_params(plan, a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc);
   p.words = static_cast<uint32_t*>(a->split_ws);
   if (a->split_ws) p.ws = reinterpret_cast<float*>(static_cast<char*>(a->split_ws) + kSplitFlagBytes);
