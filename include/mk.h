@@ -371,7 +371,9 @@ int mk_moe_permute(const mk_moe_permute_args* args, void* stream);
  *           (W: [E, K, 2I], out: [R_pad, I])   SwiGLU fused in the epilogue
  * e(r) = rb_expert[r / 128] when rb_expert is given, else the expert whose
  * padded row range [sum_{e'<e} padded[e'], sum_{e'<=e} padded[e']) holds r,
- * from padded_tokens_per_expert (the reference's own table).
+ * from padded_tokens_per_expert (the reference's own table).  Counts that sum
+ * to more than R_pad are cut off there; rows past every range go to the last
+ * expert.
  * Replaces group_gemm_fused (reference src/dispatch_gemm.cu:207-408),
  * gemm1_swiglu_fused (src/dispatch_gemm_glu_combine.cu:441-643) and
  * ffn_gemm2/grouped_gemm (src/dispatch_gemm_glu_combine.cu:247-429,647-651). */

@@ -31,6 +31,7 @@
 // the other's MFMAs).
 #include "mk_device.h"
 #include "mk_internal.h"
+#include "mk_map.h"
 #include "mk_once.h"
 #include "mk_tile.h"
 #include <mutex>
@@ -669,18 +670,13 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
           r1 += 64;
         }
       } else {
-        // the tiles whose first row is in the expert's range (the last expert
-        // also takes the rows past every range)
         int beg, end;
         const int e = expert_of_row(p, rt * C::BM, beg, end);
-        r0 = (beg + C::BM - 1) / C::BM;
-        r1 = e == p.n_experts - 1 ? tiles_m : (end + C::BM - 1) / C::BM;
+        expert_run(rt, beg, end, e == p.n_experts - 1, tiles_m, C::BM, r0, r1);
       }
       r0 = __builtin_amdgcn_readfirstlane(r0);
       r1 = __builtin_amdgcn_readfirstlane(r1);
-      const int local = t - r0 * p.tiles_n, nr = r1 - r0;
-      tn = local / nr;
-      tm = r0 + local % nr;
+      expert_run_tile(t, r0, r1, p.tiles_n, tm, tn);
     } else {
       decode_grouped(t, tiles_m, p.tiles_n, p.group_m, tm, tn);
     }

@@ -81,3 +81,35 @@ def test_grouped_gemm_orders(dev, counts, K, Nw, mode):
         # one bf16 rounding of fp32 sums in another order (and of HIP's fast exponential)
         assert torch.allclose(got, h, rtol=2 ** -7, atol=1e-4), e
         row += padded[e]
+
+
+@pytest.mark.parametrize("counts,rows", [([256, 512, 128], 512), ([256, 256, 128], 384), ([128, 384, 0, 640], 896),
+                                         ([64, 448, 512], 384), ([128, 128], 512)])
+@pytest.mark.parametrize("K,Nw,mode", [(288, 1024, 0), (256, 768, 1), (4128, 512, 0)])
+def test_grouped_gemm_counts_past_the_rows(dev, counts, rows, K, Nw, mode):
+    """Padded counts that do not sum to the launch's rows (a table built for
+    more rows than the buffers hold, or one that ends before them): every row of
+    the launch is right, and nothing behind the output is written."""
+    print(f"grouped counts={counts} rows={rows} K={K} Nw={Nw} mode={mode}", flush=True)
+    E, width, guard = len(counts), Nw // 2 if mode else Nw, 1024
+    A = wl.randn_bf16((rows + guard, K), 1, K ** -0.5).to(dev)
+    W = wl.randn_bf16((E, K, Nw), 2, K ** -0.5).to(dev)
+    ppe = torch.tensor(counts, dtype=torch.int32, device=dev)
+    rb_rows = torch.full(((rows + guard) // 128,), 128, dtype=torch.int32, device=dev)
+    total = sum(counts)
+    outs = []
+    for kw in ({}, {"rb_rows": rb_rows}, {"sizes": torch.tensor([total, max(total, rows)], dtype=torch.int64, device=dev)}):
+        out = torch.full((rows + guard, width), 7.0, dtype=torch.bfloat16, device=dev)
+        ops.moe_grouped_gemm(A[:rows], W, out[:rows], mode=mode, padded_tokens_per_expert=ppe, **kw)
+        torch.cuda.synchronize()
+        assert bool((out[rows:] == 7.0).all()), "written past the launch's rows"
+        outs.append(out[:rows])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    ends = np.cumsum(counts)
+    for r in range(0, rows, 128):  # a row tile belongs to the expert of its first row
+        e = min(int(np.searchsorted(ends, r, side="right")), E - 1)
+        h = A[r:r + 128].float().cpu() @ W[e].float().cpu()
+        if mode:
+            h = torch.nn.functional.silu(h[:, :width]) * h[:, width:]
+        # one bf16 rounding of fp32 sums in another order (and of HIP's fast exponential)
+        assert torch.allclose(outs[0][r:r + 128].float().cpu(), h, rtol=2 ** -7, atol=1e-4), r
