@@ -128,8 +128,10 @@ void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn =
   s = std::min(s, (p.K / 32) / 4);  // keep every part at >= 4 K stages
   if (bm == 256) s = mk::tail_split(R, p.K, p.n_cons, reduce, nullptr);
   if (s < 2) return;
-  const int64_t parts = (int64_t)R * (s - 1);
-  if (parts * 4 > kClaimOffset || kSplitFlagBytes + parts * bm * bn * 4 > ws_bytes) return;
+  // a partial tile for every part but one of each tile, a flag likewise (two
+  // for the two parts that swap halves)
+  const int64_t parts = (int64_t)R * (s - 1), flags = s == 2 ? 2 * R : parts;
+  if (flags * 4 > kClaimOffset || kSplitFlagBytes + parts * bm * bn * 4 > ws_bytes) return;
   p.sk_flags = static_cast<uint32_t*>(ws);
   p.sk_ws = reinterpret_cast<float*>(static_cast<char*>(ws) + kSplitFlagBytes);
   p.sk_full = ntiles - R;

@@ -1031,9 +1031,12 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
     // of the tile (one owner folding the whole tile measured ~33 us while
     // the contributor sat idle).  Each element is the sum of the same two
     // fp32 terms as with one owner (a two-term sum does not depend on order).
-    const int slot_out = tail_idx * 2 + part, slot_in = tail_idx * 2 + (1 - part);
+    // The two halves are of different waves, whose units in a partial tile are
+    // disjoint: one tile of workspace holds both.
+    const int slot_out = tail_idx * 2 + part, slot_in = tail_idx * 2 + (1 - part);  // flags
+    float* const ws = p.sk_ws + (int64_t)tail_idx * (C::BM * C::BN);
     const bool own_rows = wm == part;
-    if (!own_rows) put_partial<C>(p.sk_ws + (int64_t)slot_out * (C::BM * C::BN), acc, tid);
+    if (!own_rows) put_partial<C>(ws, acc, tid);
     // write-through stores performed at agent scope, then a relaxed flag
     // (the protocol of copy_wt: no L2 write-back needed)
     wait_vmem_all();
@@ -1045,7 +1048,7 @@ __device__ __forceinline__ void compute_role(const GemmKParams& p, int cons_id, 
     __syncthreads();
     if (own_rows) {
       // two fp32 terms: the sum is the same whichever part adds
-      add_partial_regs<C>(p.sk_ws + (int64_t)slot_in * (C::BM * C::BN), acc, tid);
+      add_partial_regs<C>(ws, acc, tid);
       store_tile<C, EPI>(p, acc, m0, tn, tid, smem);
     }
     __syncthreads();  // the partial is read: clear its flag for the next launch

@@ -95,6 +95,40 @@ def test_noalloc_tail_split_beyond_static_scratch_runs_unsplit(dev):
         assert torch.equal(full2, Ad)
 
 
+@pytest.mark.parametrize("N,rest", [(2816, 96), (3072, 128)])
+def test_noalloc_two_way_split_fits_the_static_scratch(dev, N, rest):
+    """65 to 128 tail tiles split two ways: as many partial tiles as the static
+    scratch holds at most (the piece counters lie right behind them).  Twice,
+    bit-equal to mk_ag_gemm with a full workspace, whose partial tiles past
+    those the split needs stay untouched."""
+    cus = ops.cu_count()
+    world, rows, K = 8, 1024, 4096
+    M = world * rows
+    if (M // 256) * (N // 256) != cus + rest:
+        pytest.skip("tail sizes are for 256 CUs")
+    cfg = wl.AgCfg(world=world, shard_rows=rows, K=K, N=N)
+    A, B, order = wl.ag_inputs(cfg, seed=3)
+    Ad, Bd, od = A.to(dev), B.to(dev), torch.from_numpy(order).to(dev)
+    nb = M // 128
+    ws = torch.zeros(int(capi.lib().mk_query_workspace_bytes(0, M, N, K)), dtype=torch.uint8, device=dev)
+    _say(f"noalloc two-way split N={N} tail={rest}")
+    for epoch in (4, 5):
+        full1, full2 = torch.zeros_like(Ad), torch.zeros_like(Ad)
+        flags1 = torch.zeros(nb, dtype=torch.int32, device=dev)
+        flags2, cnt1 = torch.zeros_like(flags1), torch.zeros_like(flags1)
+        C1 = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+        C2 = torch.full_like(C1, 3.0)
+        capi.call("mk_ag_gemm", _args(Ad, full1, Bd, C1, flags1, od, epoch, -1, cnt1, (ws.data_ptr(), ws.numel())),
+                  _stream())
+        capi.call("mk_ag_gemm_noalloc", _args(Ad, full2, Bd, C2, flags2, od, epoch, -1), _stream())
+        torch.cuda.synchronize()
+        assert torch.equal(C1, C2) and torch.equal(full2, Ad) and bool((flags2 == epoch).all())
+        tiles = ws[4096:].view(torch.int32).view(-1, 256 * 256)
+        written = (tiles != 0).any(1).nonzero().view(-1).tolist()
+        assert written == list(range(rest)), "a partial tile per tail tile"
+    assert rel_fro(C2[:512].float(), ag_gemm_ref(A[:512], B)) < 2e-2
+
+
 def test_noalloc_present_blocks(dev):
     """n_present through the no-alloc entry point: the own shard's blocks
     are published without a copy (junk in their source rows never reaches
