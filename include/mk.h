@@ -490,7 +490,8 @@ int mk_moe_ffn_combine(const mk_moe_ffn_args* args, void* stream);
  * shape and grid (4 KB of flag words plus one 256x256 fp32 tile per CU); `which`, M,
  * N and K are accepted for symmetry and do not change the answer.  A
  * workspace serves one launch at a time: launches that share it must be
- * ordered (same stream).  No counterpart in the reference, whose tail round
+ * ordered (same stream).  After a bounded wait gave up (bit 0 of the error
+ * word) its first 4 KB must be zeroed before the next launch that uses it.  No counterpart in the reference, whose tail round
  * simply idles (src/ag_gemm.cu:265-461). */
 int64_t mk_query_workspace_bytes(int32_t which, int64_t M, int64_t N, int64_t K);
 

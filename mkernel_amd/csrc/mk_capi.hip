@@ -108,8 +108,13 @@ int check_gemm_shape(int64_t M, int64_t N, int64_t K, int bm, int64_t lda = 0, i
 constexpr int64_t kSplitTileBytes = 256 * 256 * 4;  // one fp32 partial tile (BM x BN <= 256 x 256)
 constexpr int64_t kSplitFlagBytes = 4096;           // flag words at the start of the workspace
 // The last 64 bytes of the flag area hold the claim word of co-resident
-// staging (epoch-stamped, never reset); K-split flags use the bytes before.
+// staging (epoch-stamped, never reset).  The flags of the persistent kernel's
+// K-split and the words of the small-tile kernel's have a part of the rest
+// each: a gated launch whose bounded wait gave up can leave a flag set, and the
+// small-tile kernel, whose parts wait for each other without a bound, would
+// take a set word for a part that came.
 constexpr int64_t kClaimOffset = kSplitFlagBytes - 64;
+constexpr int64_t kSmallWordOffset = kSplitFlagBytes / 2;
 
 int64_t split_ws_bytes(int cus) { return kSplitFlagBytes + (int64_t)cus * kSplitTileBytes; }
 
@@ -131,7 +136,7 @@ void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn =
   // a partial tile for every part but one of each tile, a flag likewise (two
   // for the two parts that swap halves)
   const int64_t parts = (int64_t)R * (s - 1), flags = s == 2 ? 2 * R : parts;
-  if (flags * 4 > kClaimOffset || kSplitFlagBytes + parts * bm * bn * 4 > ws_bytes) return;
+  if (flags * 4 > kSmallWordOffset || kSplitFlagBytes + parts * bm * bn * 4 > ws_bytes) return;
   p.sk_flags = static_cast<uint32_t*>(ws);
   p.sk_ws = reinterpret_cast<float*>(static_cast<char*>(ws) + kSplitFlagBytes);
   p.sk_full = ntiles - R;
@@ -167,7 +172,8 @@ mk::GemmSmallParams small_params(const mk::GemmSmallPlan& plan, const void* A, c
 int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
   mk::GemmSmallPlan plan;
   if (!mk::plan_gemm_small(a->M, a->N, a->K, a->lda, a->ldb, cus, a->split_ws != nullptr,
-                           a->split_ws_bytes - kSplitFlagBytes, (int)(kClaimOffset / 4), {-1, 0}, &plan))
+                           a->split_ws_bytes - kSplitFlagBytes, (int)((kClaimOffset - kSmallWordOffset) / 4), {-1, 0},
+                           &plan))
     return kNoSmallPlan;
   const int64_t t256 = a->M % 256 ? 0 : (a->M / 256) * (a->N / 256);
   if (2 * t256 > cus && mk::persistent_cost(t256, a->K, cus, a->split_ws != nullptr) <= plan.us) return kNoSmallPlan;
@@ -178,8 +184,10 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
   const int64_t t128 = (a->M / 128) * (a->N / 256);
   if (a->M % 256 && a->split_ws && a->K >= 4096 && t128 > cus && 4 * t128 <= 5 * cus) return kNoSmallPlan;
   mk::GemmSmallParams p = small_params(plan, a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc);
-  p.words = static_cast<uint32_t*>(a->split_ws);
-  if (a->split_ws) p.ws = reinterpret_cast<float*>(static_cast<char*>(a->split_ws) + kSplitFlagBytes);
+  if (a->split_ws) {
+    p.words = reinterpret_cast<uint32_t*>(static_cast<char*>(a->split_ws) + kSmallWordOffset);
+    p.ws = reinterpret_cast<float*>(static_cast<char*>(a->split_ws) + kSplitFlagBytes);
+  }
   hipError_t e = mk::launch_gemm_small(p, plan, false, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? MK_OK : hip_fail(e, "mk_gemm launch");
 }
@@ -947,7 +955,7 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
     // consumer (and one flag word each).
     p.rows_dev = sizes + 1;
     p.spread_dev = num_cus <= 0 ? 1 : 0;  // the library's grid: the kernel applies the tail spread
-    if (split_ws && p.waves == 8 && (int64_t)p.n_cons * 4 <= kClaimOffset &&
+    if (split_ws && p.waves == 8 && (int64_t)p.n_cons * 4 <= kSmallWordOffset &&
         split_ws_bytes >= kSplitFlagBytes + (int64_t)p.n_cons * 128 * bn * 4) {
       p.sk_dev = 1;
       p.sk_flags = static_cast<uint32_t*>(split_ws);

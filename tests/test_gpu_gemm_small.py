@@ -90,3 +90,24 @@ def test_small_gemm_on_several_streams(dev):
     torch.cuda.synchronize()
     assert all(torch.equal(c, w) for c, w in zip(C, want))
     assert rel_fro(C[0].float(), gemm_ref(A[0].cpu(), B[0].cpu())) < 2e-2
+
+
+@pytest.mark.parametrize("M,N,K", [(640, 512, 4128), (512, 512, 4096), (1024, 512, 8192), (512, 2048, 8192)])
+def test_small_gemm_beside_flags_of_a_launch_that_gave_up(dev, M, N, K):
+    """K-split flags that a gated launch left set when its bounded wait gave up
+    (any of the words the persistent kernel uses) do not reach the small
+    kernel's own words."""
+    print(f"small gemm, set split flags, M={M} N={N} K={K}", flush=True)
+    A, B = wl.randn_bf16((M, K), 1, K ** -0.5).to(dev), wl.randn_bf16((K, N), 2, K ** -0.5).to(dev)
+    ws = torch.zeros(int(capi.lib().mk_query_workspace_bytes(0, M, N, K)), dtype=torch.uint8, device=dev)
+    want, C = (torch.empty((M, N), dtype=torch.bfloat16, device=dev) for _ in range(2))
+    _call(A, B, want, M, N, K, K, N, N, ws)
+    torch.cuda.synchronize()
+    assert bool((ws[4096:].view(torch.int32) != 0).any()), "no tile was split along K"
+    words = ws[:2048].view(torch.int32)
+    words.fill_(1)
+    for _ in range(2):
+        C.zero_()
+        _call(A, B, C, M, N, K, K, N, N, ws)
+        torch.cuda.synchronize()
+        assert torch.equal(C, want) and bool((words == 1).all()) and not bool(ws[2048:4096].any())
