@@ -20,8 +20,10 @@ def _ptr(t: torch.Tensor | None) -> int:
     return 0 if t is None else t.data_ptr()
 
 
-_raw_stream = torch._C._cuda_getCurrentRawStream  # current_stream(i).cuda_stream without the Stream object
-_device_index = torch._C._cuda_getDevice
+# current_stream(i).cuda_stream without the Stream object, where torch has these
+# (they are not part of its public interface)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda i: torch.cuda.current_stream(i).cuda_stream)
+_device_index = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _stream() -> int:

@@ -117,3 +117,21 @@ def test_entry_points_refuse_missing_arguments(name):
     assert name.encode() in L.mk_last_error_string()
     empty = _ARGS_ENTRIES[name]()  # every pointer NULL, every size 0
     assert fn(C.byref(empty), None) < 0, L.mk_last_error_string()
+
+
+def test_ops_import_without_torch_internals():
+    """mkernel_amd.ops loads, and names the current stream, on a torch that
+    lacks the two private symbols it uses where they exist."""
+    import subprocess
+    import sys
+    prog = ("import torch\n"
+            "for n in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):\n"
+            "    if hasattr(torch._C, n): delattr(torch._C, n)\n"
+            "class S: cuda_stream = 77\n"
+            "torch.cuda.current_stream = lambda *a: S\n"
+            "torch.cuda.current_device = lambda: 0\n"
+            "torch.cuda.is_initialized = lambda: True\n"
+            "from mkernel_amd import ops\n"
+            "assert ops._stream() == 77\n")
+    res = subprocess.run([sys.executable, "-c", prog], cwd=ROOT, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
