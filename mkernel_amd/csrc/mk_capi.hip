@@ -115,6 +115,11 @@ constexpr int64_t kSplitFlagBytes = 4096;           // flag words at the start o
 // take a set word for a part that came.
 constexpr int64_t kClaimOffset = kSplitFlagBytes - 64;
 constexpr int64_t kSmallWordOffset = kSplitFlagBytes / 2;
+constexpr int64_t kSmallWords = (kClaimOffset - kSmallWordOffset) / 4;
+
+uint32_t* small_words(void* split_ws) {
+  return reinterpret_cast<uint32_t*>(static_cast<char*>(split_ws) + kSmallWordOffset);
+}
 
 int64_t split_ws_bytes(int cus) { return kSplitFlagBytes + (int64_t)cus * kSplitTileBytes; }
 
@@ -172,8 +177,7 @@ mk::GemmSmallParams small_params(const mk::GemmSmallPlan& plan, const void* A, c
 int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
   mk::GemmSmallPlan plan;
   if (!mk::plan_gemm_small(a->M, a->N, a->K, a->lda, a->ldb, cus, a->split_ws != nullptr,
-                           a->split_ws_bytes - kSplitFlagBytes, (int)((kClaimOffset - kSmallWordOffset) / 4), {-1, 0},
-                           &plan))
+                           a->split_ws_bytes - kSplitFlagBytes, (int)kSmallWords, {-1, 0}, &plan))
     return kNoSmallPlan;
   const int64_t t256 = a->M % 256 ? 0 : (a->M / 256) * (a->N / 256);
   if (2 * t256 > cus && mk::persistent_cost(t256, a->K, cus, a->split_ws != nullptr) <= plan.us) return kNoSmallPlan;
@@ -185,7 +189,7 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
   if (a->M % 256 && a->split_ws && a->K >= 4096 && t128 > cus && 4 * t128 <= 5 * cus) return kNoSmallPlan;
   mk::GemmSmallParams p = small_params(plan, a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc);
   if (a->split_ws) {
-    p.words = reinterpret_cast<uint32_t*>(static_cast<char*>(a->split_ws) + kSmallWordOffset);
+    p.words = small_words(a->split_ws);
     p.ws = reinterpret_cast<float*>(static_cast<char*>(a->split_ws) + kSplitFlagBytes);
   }
   hipError_t e = mk::launch_gemm_small(p, plan, false, static_cast<hipStream_t>(stream));
@@ -193,7 +197,7 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
 }
 
 // A fused launch `p` as a sequence: the staging of its blocks on every CU, then
-// the small-tile kernel on whole tiles, then the done flags.  kNoSmallPlan: the
+// the small-tile kernel on whole tiles.  kNoSmallPlan: the
 // persistent kernel is to run; `p` then stages nothing any more if its blocks
 // were better staged first.  Every output is the same K-ordered sum on each
 // path (where the persistent kernel would split its tail along K it runs), so
@@ -212,12 +216,16 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
 // few (AllGather 4096x256x4096, world 16: 211 -> 32 with the small ones) and
 // where few rows are folded by whole workgroups (ReduceScatter 4096x4096x256,
 // world 16: 69 -> 50).
-int small_fused(mk::GemmKParams& p, bool reduce, int cus, void* stream, const char* where) {
+int small_fused(mk::GemmKParams& p, bool reduce, void* split_ws, int cus, void* stream, const char* where) {
   if (p.sk_split > 1) return kNoSmallPlan;
   const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
   mk::GemmSmallPlan plan;
   const mk::SmallFold fold{reduce ? p.rs_npeers : -1, p.rs_own_rows};
-  bool small = mk::plan_gemm_small(p.M, p.N, p.K, p.lda, p.ldb, cus, false, 0, 0, fold, &plan);
+  // the parts of a done flag's tile are counted in the workspace and stored
+  // through a buffer window of up to 128 rows
+  const bool flags = !p.ar_done || (split_ws && (int64_t)p.rs_own_rows / 256 * p.tiles_n <= kSmallWords &&
+                                    128LL * p.ldc * 2 < (1LL << 31));
+  bool small = flags && mk::plan_gemm_small(p.M, p.N, p.K, p.lda, p.ldb, cus, false, 0, 0, fold, &plan);
   if (small) {
     double one = mk::persistent_cost(tiles, p.K, cus, false), sm = plan.us;
     if (reduce) {
@@ -251,10 +259,14 @@ int small_fused(mk::GemmKParams& p, bool reduce, int cus, void* stream, const ch
   mk::GemmSmallParams q = small_params(plan, p.A, p.B, p.C, p.M, p.N, p.K, p.lda, p.ldb, p.ldc);
   q.rs_own_row0 = p.rs_own_row0; q.rs_own_rows = p.rs_own_rows; q.rs_npeers = p.rs_npeers;
   q.rs_recv = p.rs_recv; q.rs_out = p.rs_out;
+  if (p.ar_done) {
+    q.words = small_words(split_ws);
+    q.done = p.ar_done + p.rs_own_row0 / 256 * p.tiles_n;
+    q.done_cols = p.tiles_n;
+    q.epoch_ptr = p.epoch_ptr;
+    q.epoch = p.epoch;
+  }
   hipError_t e = mk::launch_gemm_small(q, plan, reduce, s);
-  if (e == hipSuccess && p.ar_done)
-    e = mk::launch_publish_done(p.ar_done + p.rs_own_row0 / 256 * p.tiles_n, p.rs_own_rows / 256 * p.tiles_n,
-                                p.epoch_ptr, p.epoch, s);
   return e == hipSuccess ? MK_OK : hip_fail(e, where);
 }
 
@@ -500,7 +512,7 @@ int prepare_ag(const mk_ag_gemm_args* a, void* stream, mk::GemmKParams& p, int* 
 
 int launch_ag(mk::GemmKParams& p, int costage, int small_cus, void* stream) {
   if (small_cus) {
-    const int rc = small_fused(p, false, small_cus, stream, "mk_ag_gemm launch");
+    const int rc = small_fused(p, false, nullptr, small_cus, stream, "mk_ag_gemm launch");
     if (rc != kNoSmallPlan) return rc;
   }
   hipError_t e = costage ? mk::launch_gemm_costaged(p, mk::kEpiStore, costage, static_cast<hipStream_t>(stream))
@@ -644,7 +656,7 @@ int rs_launch(const mk_gemm_rs_args* a, const void* peer_reduced, uint16_t* full
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, fn)) return rc;
   plan_split(p, bm, a->split_ws, a->split_ws_bytes, 256, true);
   if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
-    const int rc = small_fused(p, true, d.cus, stream, fn);
+    const int rc = small_fused(p, true, a->split_ws, d.cus, stream, fn);
     if (rc != kNoSmallPlan) return rc;
   }
   hipError_t e = costage_waves ? mk::launch_gemm_costaged(p, mk::kEpiReduce, costage_waves * total,
@@ -759,7 +771,7 @@ int mk_gemm_ar(const mk_gemm_ar_args* a, void* stream) {
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm_ar")) return rc;
   plan_split(p, bm, a->split_ws, a->split_ws_bytes, 256, true);
   if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
-    const int rc = small_fused(p, true, d.cus, stream, "mk_gemm_ar launch");
+    const int rc = small_fused(p, true, a->split_ws, d.cus, stream, "mk_gemm_ar launch");
     if (rc != kNoSmallPlan) return rc;
   }
   hipError_t e = costage_waves ? mk::launch_gemm_costaged(p, mk::kEpiReduce, costage_waves * total,

@@ -1368,18 +1368,6 @@ hipError_t launch_stage_all(const GemmKParams& p, int grid, hipStream_t stream) 
   return hipGetLastError();
 }
 
-// Every done flag of an all-reduce whose rows an earlier launch finished.
-__global__ void publish_done_kernel(uint32_t* done, int n, const uint32_t* epoch_ptr, uint32_t epoch) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n)
-    publish_flag(done + i, epoch_ptr ? __hip_atomic_load(epoch_ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : epoch);
-}
-
-hipError_t launch_publish_done(uint32_t* done, int n, const uint32_t* epoch_ptr, uint32_t epoch, hipStream_t stream) {
-  hipLaunchKernelGGL(publish_done_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, done, n, epoch_ptr, epoch);
-  return hipGetLastError();
-}
-
 hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream) {
   hipLaunchKernelGGL(epoch_advance_kernel, dim3(1), dim3(64), 0, stream, epoch_ptr);
   return hipGetLastError();

@@ -125,6 +125,24 @@ __device__ __forceinline__ void parts_in(const float* slot0, const int* where, i
     for (int b = 0; b < 4; ++b) acc[u / (C::FN * 4)][(u / 4) % C::FN][4 * (u % 4) + b] = s[u][b];
 }
 
+// One tile of a 256 x 256 tile's folded rows is stored (write-through): whoever
+// stores the last of them publishes its flag.  Relaxed atomics, as in copy_wt's
+// protocol: a release per tile (an L2 write-back) made 4096x4096x256 of world 8
+// 61 us, 50 without flags.
+template <class C>
+__device__ __forceinline__ void part_done(const GemmSmallParams& p, int row, int col, int tid) {
+  constexpr uint32_t kParts = (256 / C::BM) * (256 / C::BN);
+  wait_vmem_all();
+  __syncthreads();
+  if (tid != 0) return;
+  const int f = row / 256 * p.done_cols + col / 256;
+  if (__hip_atomic_fetch_add(p.words + f, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kParts - 1) return;
+  __hip_atomic_store(p.words + f, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t epoch =
+      p.epoch_ptr ? __hip_atomic_load(p.epoch_ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : p.epoch;
+  __hip_atomic_store(p.done + f, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <class C, bool REDUCE>
 __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -302,7 +320,8 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
     }
     if (REDUCE && m0 >= p.rs_own_row0 && m0 < p.rs_own_row0 + p.rs_own_rows) {
       static_assert(!REDUCE || C::WAVES * 32 * (C::WTN * 4 + 16) <= C::LDS_BYTES, "fold rows in LDS");
-      reduce_rows<C, 8>(p, acc, m0 - p.rs_own_row0 + wm * C::WTM, n0 + wn * C::WTN, smem, wave, lane);
+      reduce_rows<C, 8, true>(p, acc, m0 - p.rs_own_row0 + wm * C::WTM, n0 + wn * C::WTN, smem, wave, lane);
+      if (p.done) part_done<C>(p, m0 - p.rs_own_row0, n0, tid);
     } else {
       // with the fold these are the would-be sends: written once, not read here
       store_rows<C, C::FN, REDUCE>(p.C + (int64_t)(m0 + wm * C::WTM) * p.ldc + n0 + wn * C::WTN, p.ldc, acc, smem, wave,

@@ -110,9 +110,8 @@ hipError_t launch_gemm(const GemmKParams& p, int bm, int epi, hipStream_t stream
 // staging kernel runs; both claim pieces through p.st_claim.
 hipError_t launch_gemm_costaged(const GemmKParams& p, int epi, int n_stage_waves, hipStream_t stream);
 hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream);
-// The staging of p's blocks alone (st_* fields), and the done flags alone.
+// The staging of p's blocks alone (st_* fields).
 hipError_t launch_stage_all(const GemmKParams& p, int grid, hipStream_t stream);
-hipError_t launch_publish_done(uint32_t* done, int n, const uint32_t* epoch_ptr, uint32_t epoch, hipStream_t stream);
 
 // Dense GEMM of less than one round of persistent tiles (mk_gemm_small.hip).
 struct GemmSmallParams {
@@ -123,13 +122,21 @@ struct GemmSmallParams {
   int K;
   int tiles_m, tiles_n, group_m;
   int nk;            // 64-deep K stages of a tile
-  uint32_t* words;   // a ticket per tile and a header per workgroup, zero between launches
+  // zero between launches: a ticket per tile and a header per workgroup of a
+  // K-split; with done flags, the finished parts of each
+  uint32_t* words;
   float* ws;         // an fp32 tile per workgroup
   // reduce epilogue: rows rs_own_row0 .. + rs_own_rows are folded with the
   // peers' staged partials into rs_out, the others are stored to C
   int rs_own_row0, rs_own_rows, rs_npeers;
   const uint16_t* rs_recv;
   uint16_t* rs_out;
+  // flags of the folded rows' 256 x 256 tiles, row by row (null: none), each
+  // set to the epoch once all of its tile is visible at agent scope
+  uint32_t* done;
+  int done_cols;
+  const uint32_t* epoch_ptr;
+  uint32_t epoch;
 };
 struct GemmSmallPlan {
   int tile, bm, bn;  // index into the kernel's tile table, and its shape

@@ -173,8 +173,10 @@ __device__ __forceinline__ void store_rows(uint16_t* base, int64_t ldc, f32x16 (
 // adds them in rank order in fp32
 // (deterministic, one rounding) and stores 16 bytes of the owned output.
 // In the accumulator layout every load and store instruction would touch
-// 32 rows with 8 bytes each.
-template <class C, int kPeers = 4, class P>
+// 32 rows with 8 bytes each.  FLAGGED: with p.done the output goes out write-
+// through (performed at agent scope once vmcnt says it is stored, the protocol
+// of copy_wt), for a flag that needs no L2 write-back.
+template <class C, int kPeers = 4, bool FLAGGED = false, class P>
 __device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::FN], int lrow0, int col0,
                                             char* smem, int wave, int lane) {
   constexpr int PITCH = C::WTN * 4 + 16;  // bytes per LDS row (fp32)
@@ -188,6 +190,10 @@ __device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::
   const int rr = l / LPR, cc = l % LPR;
   const int64_t peer_stride = (int64_t)p.rs_own_rows * p.ldc;
   const int np = p.rs_npeers;
+  // the wave's rows, from its first column on
+  const __amdgpu_buffer_rsrc_t out = make_rsrc(
+      p.rs_out + (int64_t)__builtin_amdgcn_readfirstlane(lrow0) * p.ldc + __builtin_amdgcn_readfirstlane(col0),
+      (uint32_t)(((C::WTM - 1) * p.ldc + C::WTN) * 2));
 #pragma unroll
   for (int i = 0; i < C::FM; ++i) {
 #pragma unroll
@@ -238,6 +244,12 @@ __device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::
       uint4 o;
       o.x = pack_bf16x2(x[0], x[1]); o.y = pack_bf16x2(x[2], x[3]);
       o.z = pack_bf16x2(x[4], x[5]); o.w = pack_bf16x2(x[6], x[7]);
+      if constexpr (FLAGGED)
+        if (p.done) {
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{o.x, o.y, o.z, o.w}, out,
+                                                 (int)(((i * 32 + row) * p.ldc + cc * 8) * 2), 0, 0x10 /* SC1 */);
+          continue;
+        }
       typedef uint32_t nt_u32x4 __attribute__((ext_vector_type(4)));
       __builtin_nontemporal_store(nt_u32x4{o.x, o.y, o.z, o.w},
                                   reinterpret_cast<nt_u32x4*>(p.rs_out + (int64_t)(lrow0 + i * 32 + row) * p.ldc +

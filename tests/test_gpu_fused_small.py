@@ -1,11 +1,13 @@
 """AllGather / ReduceScatter / AllReduce launches that stage first and then run
 the small-tile kernel, against the persistent kernel (the same call with the
 grid named) and the oracle: bit-equal outputs, staged bytes, flags."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from mkernel_amd import ops, workloads as wl
+from mkernel_amd import capi, ops, workloads as wl
 from oracle.gemm import gemm_ref
 
 pytestmark = pytest.mark.gpu
@@ -118,3 +120,55 @@ def test_ar_two_shot_small(dev, world, rank, M, N, K):
     per = N // 256
     assert bool((done[lo // 256 * per:hi // 256 * per] == 9).all())
     assert int((done != 0).sum()) == s // 256 * per
+
+
+@pytest.mark.parametrize("world,M,N,K,two_shot", [(4, 512, 512, 64, False), (8, 2048, 1024, 992, False),
+                                                  (2, 2560, 768, 160, False), (16, 4096, 4096, 256, True),
+                                                  (8, 2048, 2304, 32, True), (2, 1024, 1024, 544, True)])
+def test_done_flags_come_from_the_tiles(dev, world, M, N, K, two_shot):
+    """Done flags are published by the launch that folds the tiles, not by one
+    behind it, under several epochs (the parts are counted in the workspace,
+    which is left zeroed), and without a workspace too."""
+    print(f"done flags world={world} M={M} N={N} K={K} two_shot={two_shot}", flush=True)
+    A, B = wl.randn_bf16((M, K), 8, K ** -0.5).to(dev), wl.randn_bf16((K, N), 9, K ** -0.5).to(dev)
+    rows, rank = (M // world, world - 1) if two_shot else (M, 0)
+    peers = wl.randn_bf16((world - 1, rows, N), 10, 0.5).to(dev)
+    reduced = wl.randn_bf16((world - 1, rows, N), 11, 0.5).to(dev)
+    n = (world - 1) * rows // 128 * (1 + two_shot)
+    ws = torch.zeros(int(capi.lib().mk_query_workspace_bytes(0, M, N, K)), dtype=torch.uint8, device=dev)
+    flags, counters, done = _words(n, dev), _words(n, dev), _words((M // 256) * (N // 256), dev)
+    recv = torch.zeros_like(peers)
+    C, sends = (torch.empty((M, N), dtype=torch.bfloat16, device=dev) for _ in range(2))
+    epoch = torch.full((1,), 3, dtype=torch.int32, device=dev)
+
+    def call(ws, done, **kw):
+        if two_shot:
+            ops.gemm_ar_two_shot(A, B, C, sends, peers, recv, reduced, world, rank, flags, None, epoch=1,
+                                 stage_counters=counters, done_flags=done, split_ws=ws, **kw)
+        else:
+            ops.gemm_ar(A, B, C, peers, recv, world, flags, None, epoch=1, stage_counters=counters, done_flags=done,
+                        split_ws=ws, **kw)
+
+    lo, hi = rank * rows // 256 * (N // 256), (rank + 1) * rows // 256 * (N // 256)
+    outs = []
+    for split in (ws, ws, False):
+        epoch += 1
+        done.zero_()
+        call(split, done, epoch_ptr=epoch)
+        torch.cuda.synchronize()
+        assert bool((done[lo:hi] == epoch).all()) and int((done != 0).sum()) == hi - lo
+        assert not bool(ws[:4096].any())
+        outs.append(C.clone())
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert _graph_nodes(lambda: call(ws, done, epoch_ptr=epoch)) == _graph_nodes(lambda: call(ws, None, epoch_ptr=epoch))
+
+
+def _graph_nodes(call):
+    """Nodes of the graph that `call` is captured into."""
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        call()
+    n = ctypes.c_size_t(0)
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
