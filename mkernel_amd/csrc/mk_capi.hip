@@ -913,13 +913,13 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
   p.lda = K; p.ldb = Nw; p.ldc = mode == 1 ? Nw / 2 : Nw;
   p.b_expert_stride = K * Nw;
   p.M = (int)R_pad; p.N = (int)Nw; p.K = (int)K;
-  // 128 x 512 tiles stream each expert's activation rows half as often per
-  // weight byte as 128 x 256 tiles.  A handful of row blocks with a long K
-  // (at most 10, or with a device row count a capacity of fewer than 256 routed
-  // rows) makes too few of them to stream at the chip's rate: us at 512 / 256
-  // columns, K 7168, 2 blocks 56 / 43, 6 90 / 75, 9 120 / 116, 13 143 / 148.
-  const bool few = K >= mk::kExpertSplitK && (sizes ? R_pad - 127LL * E < 256 : R_pad / 128 <= 10);
+  // tile width: see few_row_blocks.  R_pad bounds the row blocks of a launch
+  // with a device row count, whose kernel makes the choice where more may come
+  // (64 experts of 7168 x 4096 in 64 blocks of capacity, SwiGLU: 731 us with the
+  // narrow tiles, 622 with the wide ones).
+  const bool few = mk::few_row_blocks(R_pad / 128, K);
   const int bn = tile_n ? tile_n : (Nw % 512 == 0 && !few ? 512 : 256);
+  const bool dev_bn = sizes && !tile_n && bn == 512 && mk::few_row_blocks(1, K);
   p.tiles_m = (int)(R_pad / 128);
   p.tiles_n = (int)(Nw / bn);
   p.rb_expert = rb_expert;
@@ -933,7 +933,7 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
   p.gather_devs = devs_per_node;
   int total;
   if (int rc = grid_total(num_cus, d, "mk_moe_grouped_gemm", &total)) return rc;
-  set_grid(p, total, 0, p.tiles_m * p.tiles_n);
+  set_grid(p, total, 0, p.tiles_m * p.tiles_n * (dev_bn ? 2 : 1));
   // Each expert's tiles together, column-major inside its run of row tiles: an
   // expert's activation rows are fetched once per XCD and its row tiles share
   // each weight slice.  GEMM1 + SwiGLU against walking all row tiles of one
@@ -976,7 +976,8 @@ static int grouped_gemm_impl(const void* A, const void* W, void* out, const int3
   } else if (split_k) {
     plan_split(p, 128, split_ws, split_ws_bytes, bn);
   }
-  hipError_t e = mk::launch_gemm(p, 128, mode == 1 ? mk::kEpiSwiGLU : mk::kEpiStore, stream, bn);
+  const int epi = mode == 1 ? mk::kEpiSwiGLU : mk::kEpiStore;
+  hipError_t e = dev_bn && p.waves == 8 ? mk::launch_gemm_expert(p, epi, stream) : mk::launch_gemm(p, 128, epi, stream, bn);
   return e == hipSuccess ? MK_OK : hip_fail(e, "mk_moe_grouped_gemm launch");
 }
 

@@ -34,6 +34,7 @@
 #include "mk_map.h"
 #include "mk_once.h"
 #include "mk_tile.h"
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -1342,6 +1343,18 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gemm_kernel(GemmKParams p) {
   gemm_main<BM, WAVES, EPI, BN>(p);
 }
 
+// Expert GEMM at a row capacity: 128 x 512 tiles (tiles_n counts those), or
+// 128 x 256 when the device's row count turns out to be a handful of blocks.
+template <int EPI>
+__global__ __launch_bounds__(512, 1) void gemm_expert_kernel(GemmKParams p) {
+  if (few_row_blocks(*p.rows_dev / 128, p.K)) {
+    p.tiles_n *= 2;
+    gemm_main<128, 8, EPI, 256>(p);
+  } else {
+    gemm_main<128, 8, EPI, 512>(p);
+  }
+}
+
 // The 256 x 256 GEMM that runs beside the staging kernel, capped at 224
 // VGPRs per wave (the attribute counts in units of two registers on gfx950,
 // whose waves draw VGPRs and AGPRs from one 512-entry file per SIMD lane):
@@ -1376,25 +1389,35 @@ hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream) {
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
-template <int BM, int WAVES, int EPI, int BN>
-static hipError_t launch_t(const GemmKParams& p, hipStream_t stream) {
-  using C = Cfg<BM, WAVES, BN>;
+template <void (*KERNEL)(GemmKParams)>
+static hipError_t launch_k(const GemmKParams& p, int threads, uint32_t lds, hipStream_t stream) {
   // The dynamic-LDS limit is raised once per device and kernel.  Two
   // threads that both find the flag clear both set the attribute, which is
   // harmless; a launch never runs before its device's attribute is set.
   static PerDeviceFlag attr_set;
-  constexpr uint32_t lds = C::LDS_BYTES;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (!attr_set.is_set(dev)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<BM, WAVES, EPI, BN>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
     attr_set.set(dev);
   }
-  hipLaunchKernelGGL((gemm_kernel<BM, WAVES, EPI, BN>), dim3(p.n_prod + p.n_cons), dim3(C::NT), lds, stream, p);
+  hipLaunchKernelGGL(KERNEL, dim3(p.n_prod + p.n_cons), dim3(threads), lds, stream, p);
   return hipGetLastError();
+}
+
+template <int BM, int WAVES, int EPI, int BN>
+static hipError_t launch_t(const GemmKParams& p, hipStream_t stream) {
+  using C = Cfg<BM, WAVES, BN>;
+  return launch_k<gemm_kernel<BM, WAVES, EPI, BN>>(p, C::NT, C::LDS_BYTES, stream);
+}
+
+hipError_t launch_gemm_expert(const GemmKParams& p, int epi, hipStream_t stream) {
+  constexpr uint32_t lds = std::max(Cfg<128, 8, 256>::LDS_BYTES, Cfg<128, 8, 512>::LDS_BYTES);
+  if (p.waves != 8 || !p.rows_dev || (epi != kEpiStore && epi != kEpiSwiGLU)) return hipErrorInvalidValue;
+  return epi == kEpiStore ? launch_k<gemm_expert_kernel<kEpiStore>>(p, 512, lds, stream)
+                          : launch_k<gemm_expert_kernel<kEpiSwiGLU>>(p, 512, lds, stream);
 }
 
 template <int BM, int EPI>

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mk_map.h"
+
 namespace mk {
 
 enum Epilogue : int { kEpiStore = 0, kEpiSwiGLU = 1, kEpiReduce = 2 };
@@ -12,13 +14,6 @@ constexpr int kMaxTilesM = 512;
 constexpr int kMaxSplitListTiles = 4096;  // K-split with a permuted tile order: at most this many tiles
 constexpr int kMaxRounds = 64;   // cooperative staging between rounds: at most this many rounds
 constexpr int kPieces = 16;  // cooperative staging: pieces per 128-row block
-
-// Expert GEMMs split a tail tile along K from this K on.  The parts' exchange
-// takes 20 to 30 us: a third of a tile's time at K 7168 (6 experts of 4096
-// columns, 48 tiles: 155 us whole, 92 split), more than it saves at 2048 (280
-// tiles: 134 us with the 24 of the tail split, 114 on 144 workgroups; 84
-// tiles: 40 whole, 51 split).
-constexpr int kExpertSplitK = 4096;
 
 struct GemmKParams {
   // operands
@@ -105,6 +100,9 @@ struct GemmKParams {
 };
 
 hipError_t launch_gemm(const GemmKParams& p, int bm, int epi, hipStream_t stream, int bn = 256);
+// Expert GEMM with a device row count, which the tile width follows
+// (few_row_blocks); p.tiles_n counts 512-column tiles.
+hipError_t launch_gemm_expert(const GemmKParams& p, int epi, hipStream_t stream);
 // Co-resident staging: the one-wave staging kernel (waves_per_cu per CU)
 // followed by a register-capped 256 x 256 GEMM that may start while the
 // staging kernel runs; both claim pieces through p.st_claim.

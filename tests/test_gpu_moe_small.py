@@ -113,3 +113,39 @@ def test_grouped_gemm_counts_past_the_rows(dev, counts, rows, K, Nw, mode):
             h = torch.nn.functional.silu(h[:, :width]) * h[:, width:]
         # one bf16 rounding of fp32 sums in another order (and of HIP's fast exponential)
         assert torch.allclose(outs[0][r:r + 128].float().cpu(), h, rtol=2 ** -7, atol=1e-4), r
+
+
+@pytest.mark.parametrize("blocks", [16, 12, 11, 10, 3, 0])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_tile_width_follows_the_device_rows(dev, blocks, mode):
+    """With a device row count the tile width follows the row blocks that are
+    there, however tight the capacity: bit-equal to the wide tiles above 10
+    blocks, to the narrow ones up to 10.  (K is split differently there.)"""
+    print(f"tile width blocks={blocks} mode={mode}", flush=True)
+    E, K, Nw = 16, 4128, 4096
+    g = torch.Generator(device=dev).manual_seed(blocks)
+    A = torch.randn((E * 128, K), generator=g, device=dev).mul_(K ** -0.5).to(torch.bfloat16)
+    W = torch.empty((E, K, Nw), dtype=torch.bfloat16, device=dev)
+    for e in range(E):
+        W[e] = torch.randn((K, Nw), generator=g, device=dev).mul_(K ** -0.5)
+    rb = torch.arange(E, dtype=torch.int32, device=dev)
+    sizes = torch.tensor([blocks * 128, blocks * 128], dtype=torch.int64, device=dev)
+    width = Nw // 2 if mode else Nw
+    outs = {}
+    for tile_n in (0, 256, 512):
+        for ws in (None, False):
+            out = torch.full((E * 128, width), 7.0, dtype=torch.bfloat16, device=dev)
+            ops.moe_grouped_gemm(A, W, out, rb_expert=rb, mode=mode, sizes=sizes, tile_n=tile_n, split_ws=ws)
+            torch.cuda.synchronize()
+            assert bool((out[blocks * 128:] == 7.0).all())
+            outs[tile_n, ws] = out
+    assert torch.equal(outs[0, None], outs[256 if blocks <= 10 else 512, None])
+    if blocks >= 10:
+        assert not torch.equal(outs[256, None], outs[512, None]), "the widths are told apart by their K-split"
+    for b in range(blocks):
+        h = A[b * 128:(b + 1) * 128].float() @ W[b].float()
+        if mode:
+            h = torch.nn.functional.silu(h[:, :width]) * h[:, width:]
+        # one bf16 rounding of fp32 sums in another order (and of HIP's fast exponential)
+        for out in (outs[0, None], outs[0, False]):
+            assert torch.allclose(out[b * 128:(b + 1) * 128].float(), h, rtol=2 ** -7, atol=1e-4), b
