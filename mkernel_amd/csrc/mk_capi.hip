@@ -124,19 +124,15 @@ uint32_t* small_words(void* split_ws) {
 int64_t split_ws_bytes(int cus) { return kSplitFlagBytes + (int64_t)cus * kSplitTileBytes; }
 
 // K-split plan for the tail round: with R = tiles % n_cons tiles left for a
-// partial last round, split each of them s ways along K so that R*s workgroups
-// share the round: as many as fit, up to 4, for the expert GEMMs, which stream
-// weights; as tail_split finds best for dense 256-row tiles.  The workspace holds the flag
-// words at a fixed offset (so every plan finds them zeroed) followed by
+// partial last round, split each of them s = tail_parts ways along K so that
+// R*s workgroups share the round.  The workspace holds the flag words at a fixed offset (so every plan finds them zeroed) followed by
 // R*(s-1) < n_cons <= CUs partial tiles, which split_ws_bytes covers.
 void plan_split(mk::GemmKParams& p, int bm, void* ws, int64_t ws_bytes, int bn = 256, bool reduce = false) {
   const int ntiles = p.tiles_m * p.tiles_n;
   const int R = ntiles % p.n_cons;
   if (!ws || R == 0 || p.waves != 8) return;
   if (p.perm_mode != mk::kPermNone && ntiles > mk::kMaxSplitListTiles) return;
-  int s = std::min(4, p.n_cons / R);
-  s = std::min(s, (p.K / 32) / 4);  // keep every part at >= 4 K stages
-  if (bm == 256) s = mk::tail_split(R, p.K, p.n_cons, reduce, nullptr);
+  const int s = mk::tail_parts(R, p.K, bm, p.n_cons, reduce);
   if (s < 2) return;
   // a partial tile for every part but one of each tile, a flag likewise (two
   // for the two parts that swap halves)
@@ -172,21 +168,11 @@ mk::GemmSmallParams small_params(const mk::GemmSmallPlan& plan, const void* A, c
   return p;
 }
 
-// C = A @ B by the small-tile kernel.  kNoSmallPlan: none of its tiles fits,
-// or the persistent kernel's 256-row tiles do and are estimated to be faster.
+// C = A @ B by the small-tile kernel, or kNoSmallPlan: the persistent kernel's.
 int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
   mk::GemmSmallPlan plan;
-  if (!mk::plan_gemm_small(a->M, a->N, a->K, a->lda, a->ldb, cus, a->split_ws != nullptr,
-                           a->split_ws_bytes - kSplitFlagBytes, (int)kSmallWords, {-1, 0}, &plan))
-    return kNoSmallPlan;
-  const int64_t t256 = a->M % 256 ? 0 : (a->M / 256) * (a->N / 256);
-  if (2 * t256 > cus && mk::persistent_cost(t256, a->K, cus, a->split_ws != nullptr) <= plan.us) return kNoSmallPlan;
-  // An odd number of 128-row blocks, a little over one round of 128 x 256 tiles
-  // and a long K: the persistent kernel splits the few tiles of the second
-  // round four ways (4224x2048x5504, 264 tiles: 119 us, 123 in two rounds of
-  // small tiles; at K 3072, 261 tiles: 77 and 75).
-  const int64_t t128 = (a->M / 128) * (a->N / 256);
-  if (a->M % 256 && a->split_ws && a->K >= 4096 && t128 > cus && 4 * t128 <= 5 * cus) return kNoSmallPlan;
+  const mk::SmallSpace ws = {a->split_ws ? kSmallWords : 0, a->split_ws ? a->split_ws_bytes - kSplitFlagBytes : 0};
+  if (!mk::gemm_runs_small(a->M, a->N, a->K, a->lda, a->ldb, cus, ws, &plan)) return kNoSmallPlan;
   mk::GemmSmallParams p = small_params(plan, a->A, a->B, a->C, a->M, a->N, a->K, a->lda, a->ldb, a->ldc);
   if (a->split_ws) {
     p.words = small_words(a->split_ws);
@@ -196,67 +182,33 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
   return e == hipSuccess ? MK_OK : hip_fail(e, "mk_gemm launch");
 }
 
-// A fused launch `p` as a sequence: the staging of its blocks on every CU, then
-// the small-tile kernel on whole tiles.  kNoSmallPlan: the
-// persistent kernel is to run; `p` then stages nothing any more if its blocks
-// were better staged first.  Every output is the same K-ordered sum on each
-// path (where the persistent kernel would split its tail along K it runs), so
-// results do not depend on how the blocks arrive.  Not for flags that someone
-// else publishes: those must be able to arrive while the launch waits.
-//
-// The persistent kernel's workgroups copy between their tiles, which hides
-// part of the copy behind others' tiles when there are several rounds and a
-// round is longer than its share of the copy.  Staging first was faster (us,
-// in the launch -> first) for AllGather below two rounds (12288x1280x2784 114
-// -> 100) or K 2048 (16384x3584x1024 146 -> 138; 16384x3584x8192 805 -> 812)
-// and for ReduceScatter below K 1024 (16384x8192, world 8: K 512 321 -> 233,
-// 1536 453 -> 449, 3584 865 -> 871); the all-reduces, whose fold or second
-// copy is spread over all rounds, gained nothing (8192^2, two-shot, K 768 171
-// -> 179).  The tiles of the persistent kernel are too large where there are
-// few (AllGather 4096x256x4096, world 16: 211 -> 32 with the small ones) and
-// where few rows are folded by whole workgroups (ReduceScatter 4096x4096x256,
-// world 16: 69 -> 50).
+// A fused launch `p` as plan_fused has it.  kNoSmallPlan: the persistent kernel
+// is to run; `p` then stages nothing any more if its blocks were staged first.
+// Where that kernel would split its tail along K it runs, so that results do not
+// depend on how the blocks arrive.  Not for flags that someone else publishes:
+// those must be able to arrive while the launch waits.
 int small_fused(mk::GemmKParams& p, bool reduce, void* split_ws, int cus, void* stream, const char* where) {
   if (p.sk_split > 1) return kNoSmallPlan;
-  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-  mk::GemmSmallPlan plan;
-  const mk::SmallFold fold{reduce ? p.rs_npeers : -1, p.rs_own_rows};
   // the parts of a done flag's tile are counted in the workspace and stored
   // through a buffer window of up to 128 rows
   const bool flags = !p.ar_done || (split_ws && (int64_t)p.rs_own_rows / 256 * p.tiles_n <= kSmallWords &&
                                     128LL * p.ldc * 2 < (1LL << 31));
-  bool small = flags && mk::plan_gemm_small(p.M, p.N, p.K, p.lda, p.ldb, cus, false, 0, 0, fold, &plan);
-  if (small) {
-    double one = mk::persistent_cost(tiles, p.K, cus, false), sm = plan.us;
-    if (reduce) {
-      // a workgroup of the persistent kernel folds in about two of its rounds
-      // when the last is not full; either kernel moves its stores and partials
-      // at 2.5 TB/s at most
-      const double bytes = 2.0 * p.N * ((double)p.M + (double)p.rs_npeers * p.rs_own_rows) / 2.5e6;
-      const bool partial = tiles > cus && tiles % cus;
-      one += (partial ? 2.0 : 1.0) * mk::fold_cost(fold, (double)p.rs_own_rows / 256 * p.tiles_n, 65536.0, cus);
-      one = std::max(one, bytes) + (partial ? 14.0 : 7.0);
-      sm = std::max(sm, bytes) + 8.0;
-    }
-    small = sm < one;
-  }
-  const bool first = p.st_nblocks > 0 &&
-                     (small || (reduce ? p.K < 1024 && !p.st_src2 && p.rs_own_rows < p.M
-                                       : tiles < 2 * cus || p.K < 2048));
+  const mk::FusedPlan f = mk::plan_fused(p.M, p.N, p.K, p.lda, p.ldb, cus, {reduce ? p.rs_npeers : -1, p.rs_own_rows},
+                                         p.st_nblocks, p.st_src2 != nullptr, flags);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (first) {
+  if (f.first) {
     hipError_t e = mk::launch_stage_all(p, std::min(p.st_nblocks * mk::kPieces, 8 * cus), s);
     if (e != hipSuccess) return hip_fail(e, where);
   }
-  if (!small) {
-    if (first) {
+  if (!f.small) {
+    if (f.first) {
       // the flags are published: the launch gates on them without a wait
       p.st_nblocks = 0;
       p.st_coop = 0;
     }
     return kNoSmallPlan;
   }
-  mk::GemmSmallParams q = small_params(plan, p.A, p.B, p.C, p.M, p.N, p.K, p.lda, p.ldb, p.ldc);
+  mk::GemmSmallParams q = small_params(f.plan, p.A, p.B, p.C, p.M, p.N, p.K, p.lda, p.ldb, p.ldc);
   q.rs_own_row0 = p.rs_own_row0; q.rs_own_rows = p.rs_own_rows; q.rs_npeers = p.rs_npeers;
   q.rs_recv = p.rs_recv; q.rs_out = p.rs_out;
   if (p.ar_done) {
@@ -266,7 +218,7 @@ int small_fused(mk::GemmKParams& p, bool reduce, void* split_ws, int cus, void* 
     q.epoch_ptr = p.epoch_ptr;
     q.epoch = p.epoch;
   }
-  hipError_t e = mk::launch_gemm_small(q, plan, reduce, s);
+  hipError_t e = mk::launch_gemm_small(q, f.plan, reduce, s);
   return e == hipSuccess ? MK_OK : hip_fail(e, where);
 }
 

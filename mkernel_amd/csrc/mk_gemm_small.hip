@@ -347,115 +347,7 @@ hipError_t launch_s(const GemmSmallParams& p, int grid, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The tile shapes and what they cost, in us.  A launch of g tiles runs in
-// rounds of per_cu x CUs workgroups (what fits the LDS of a CU together), each
-//   round + stages x slope(x),   x = the round's workgroups per CU,
-// slope = one + load x while no CU holds two, else two + more (x - 1): a full
-// chip clocks lower and shares its caches.  `start` comes once, `meet` when
-// the parts of a tile have to meet.  Fitted to N(0, 1/K) operands at 40 shapes
-// of 128 .. 10240 rows, 256 .. 8192 columns and 256 .. 8192 K on one MI355X.
-// The two-stage rings (128 x 128 at 64 KB, 64 x 64 at 32 KB) hide one tile's
-// first loads and its store behind its neighbours on the CU, which is worth
-// more than a deeper ring when many short tiles follow each other:
-// 10240x6656x512 takes 82 us with them, 107 with one 128 KB ring per CU.
-struct TileCost {
-  int bm, bn, per_cu;
-  double start, round, one, load, two, more, meet;
-};
-constexpr TileCost kTiles[] = {
-    {64, 64, 3, 1.8, 1.2, 0.235, 0.0, 0.33, 0.125, 7.0},
-    {128, 64, 2, 0.7, 1.6, 0.380, 0.0, 0.60, 0.02, 7.0},
-    {128, 128, 1, 3.0, 1.0, 0.410, 0.14, 0.0, 0.0, 10.0},
-    {192, 128, 1, 3.0, 2.0, 0.470, 0.33, 0.0, 0.0, 10.0},
-    {128, 256, 1, 2.5, 2.3, 0.620, 0.28, 0.0, 0.0, 14.0},
-    {128, 128, 2, 3.0, 2.0, 0.530, 0.05, 0.717, 0.245, 10.0},
-    {64, 64, 5, 0.8, 2.2, 0.300, 0.0, 0.31, 0.155, 7.0},
-};
-// The 32 KB ring of the last: its many workgroups hide a fold's loads
-// (ReduceScatter 4096x4096x256, world 16: 27 us against 32), but a plain
-// product of tall tiles thrashes L2 with them (5504x768x896 18.5 us, 14.5 with
-// the 128 x 128 tiles at 64 KB).
-constexpr int kFoldOnly = 5;
-
-double rounds_cost(const TileCost& c, int64_t g, double stages, int cus) {
-  const int64_t full = (int64_t)c.per_cu * cus;
-  auto round = [&](int64_t n) {
-    const double x = (double)n / cus;
-    return c.round + stages * (n > cus ? c.two + c.more * (x - 1) : c.one + c.load * x);
-  };
-  return c.start + (double)(g / full) * round(full) + (g % full ? round(g % full) : 0.0);
-}
-
 }  // namespace
-
-bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int cus, bool ws, int64_t ws_tiles_bytes,
-                     int ws_words, const SmallFold& fold, GemmSmallPlan* plan) {
-  // offsets from 2^31 up read as zeros, so both buffer windows end below it
-  if (K * ldb * 2 >= (1LL << 31)) return false;
-  const int64_t nk = (K + 63) / 64;
-  const bool reduce = fold.peers >= 0;
-  bool found = false;
-  for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
-    const TileCost& c = kTiles[i];
-    if (c.per_cu == kFoldOnly && !reduce) continue;
-    if (M % c.bm || N % c.bn || (reduce && 256 % c.bm) || (int64_t)c.bm * lda * 2 >= (1LL << 31)) continue;
-    const int64_t nt = (M / c.bm) * (N / c.bn);
-    if (nt * nk >= (1LL << 31)) continue;
-    for (int s = 1; s <= 4; ++s) {
-      const int64_t g = nt * s;
-      if (s > 1 && (!ws || reduce || g > cus || nk < 4 * s || nt + g > ws_words ||
-                    g * c.bm * c.bn * 4 > ws_tiles_bytes))
-        break;
-      double t = rounds_cost(c, g, (double)((nk + s - 1) / s), cus) + (s > 1 ? c.meet : 0.0);
-      if (reduce) t += fold_cost(fold, (double)fold.rows / c.bm * (N / c.bn), (double)c.bm * c.bn, c.per_cu * cus);
-      if (!found || t < plan->us) {
-        found = true;
-        *plan = {i, c.bm, c.bn, (int)g, s, t};
-      }
-    }
-  }
-  return found;
-}
-
-namespace {
-double persistent_round(double tiles, double stages, int cus) { return 3.8 + stages * (0.24 + 0.55 * tiles / cus); }
-}  // namespace
-
-int tail_split(int64_t rest, int64_t K, int cus, bool reduce, double* us) {
-  const double stages = (double)K / 32;
-  int best = 1;
-  double t = persistent_round((double)rest, stages, cus);
-  for (int s = 2; s <= 4 && rest * s <= cus && K / 32 >= 4 * s; ++s) {
-    const double ts = persistent_round((double)(rest * s), stages / s, cus) + (reduce ? 80.0 : 10.0 + 1.5 * s);
-    if (ts < t) {
-      t = ts;
-      best = s;
-    }
-  }
-  if (us) *us = t;
-  return best;
-}
-
-double persistent_cost(int64_t tiles, int64_t K, int cus, bool split) {
-  const double stages = (double)K / 32;
-  double t = 5.0 + (double)(tiles / cus) * persistent_round(cus, stages, cus);
-  const int64_t rest = tiles % cus;
-  if (rest && split && tiles > cus) {
-    double tail;
-    tail_split(rest, K, cus, false, &tail);
-    t += tail;
-  } else if (rest) {
-    t += persistent_round((double)rest, stages, cus);
-  }
-  return t;
-}
-
-double fold_cost(const SmallFold& f, double tiles, double tile_elems, double at_once) {
-  if (f.peers <= 0) return 0.0;
-  const double chip = tiles * tile_elems * 2 * f.peers / 7e6, one = tile_elems * 2 * f.peers / 0.06e6;
-  const double own = one * (double)(int64_t)((tiles + at_once - 1) / at_once);
-  return chip > own ? chip : own;
-}
 
 hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, bool reduce, hipStream_t stream) {
   const int grid = plan.grid;

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "mk_map.h"
+#include "mk_plan.h"
 
 namespace mk {
 
@@ -111,7 +112,7 @@ hipError_t launch_epoch_advance(uint32_t* epoch_ptr, hipStream_t stream);
 // The staging of p's blocks alone (st_* fields).
 hipError_t launch_stage_all(const GemmKParams& p, int grid, hipStream_t stream);
 
-// Dense GEMM of less than one round of persistent tiles (mk_gemm_small.hip).
+// Dense GEMM on small tiles (mk_gemm_small.hip).
 struct GemmSmallParams {
   const uint16_t* A;
   const uint16_t* B;
@@ -136,39 +137,6 @@ struct GemmSmallParams {
   const uint32_t* epoch_ptr;
   uint32_t epoch;
 };
-struct GemmSmallPlan {
-  int tile, bm, bn;  // index into the kernel's tile table, and its shape
-  int grid, split;   // workgroups, and parts of each tile along K
-  double us;         // estimated time
-};
-// The fold of a reduce epilogue: `rows` rows with `peers` partials each
-// (peers < 0: no such epilogue).
-struct SmallFold {
-  int peers;
-  int64_t rows;
-};
-// Estimated us of folding `tiles` tiles, `at_once` workgroups at a time: the
-// chip takes 7 TB/s of partials beside its products, one workgroup 60 GB/s.
-double fold_cost(const SmallFold& f, double tiles, double tile_elems, double at_once);
-// The tile and split with the least estimated time; false: no tile fits.
-// ws: a workspace of ws_words words and ws_tiles_bytes of tiles is there.
-bool plan_gemm_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int cus, bool ws, int64_t ws_tiles_bytes,
-                     int ws_words, const SmallFold& fold, GemmSmallPlan* plan);
-// Parts along K (1..4) for `rest` 256 x 256 tiles of a last round on `cus`
-// workgroups, and its estimated us: splitting fills the idle CUs, which then
-// clock lower, and costs the parts' exchange, about 13 us for two of them.
-// Measured, whole against split tail: 10240x2048x1024 (64 tiles) 54 against
-// 80 us, 16384x6656x416 (128) 122 against 137, 16384x3584x3584 (128) equal,
-// 9216x2048x3584 (32) 153 against 146, 16384x3584x8192 (128) 745 against 735.
-// With the reduce epilogue the exchange costs 35 to 90 us (its registers spill
-// beside the fold: 16384x3584x3584, 128 tiles, 406 whole and 480 split with the
-// partials staged in the launch; 10240x2048x1024, 64 tiles, 84 and 127), so
-// only a K of about 14000 and more is split there.
-int tail_split(int64_t rest, int64_t K, int cus, bool reduce, double* us);
-// Estimated us of the persistent kernel on `tiles` 256 x 256 tiles (split:
-// with a workspace for the K-split of its tail).  Fitted like the tile table:
-// 4096^3 106-118 measured, 8192x8192x512 71, 8192x3584x8192 382.
-double persistent_cost(int64_t tiles, int64_t K, int cus, bool split);
 hipError_t launch_gemm_small(const GemmSmallParams& p, const GemmSmallPlan& plan, bool reduce, hipStream_t stream);
 
 struct PermuteKParams {

@@ -12,6 +12,20 @@ from oracle.gemm import gemm_ref
 
 pytestmark = pytest.mark.gpu
 
+# every tile shape that each operation may get, and blocks staged first before
+# the persistent kernel (the last of AG and of RS); tests/test_plans.py says so
+AG = [(2, 512, 256, 32, 0), (16, 4096, 256, 1056, 2), (4, 2048, 512, 992, 4), (8, 4096, 1024, 512, 0),
+      (1, 256, 768, 96, 2), (3, 768, 512, 4128, 0), (2, 1536, 2816, 288, 3), (2, 3584, 1792, 160, 0),
+      (4, 7168, 1792, 32, 0), (4, 5120, 3328, 32, 1), (16, 20480, 1536, 32, 0)]
+RS = [(2, 1, 512, 256, 32), (16, 5, 4096, 4096, 256), (4, 0, 2048, 768, 416), (1, 0, 512, 512, 96),
+      (8, 7, 2048, 1024, 2080), (2, 0, 1536, 2304, 160), (8, 3, 2048, 256, 32), (4, 2, 5120, 3328, 32),
+      (2, 1, 3584, 1792, 160), (8, 0, 10240, 1280, 32), (8, 6, 6144, 256, 32), (2, 1, 2560, 3584, 32)]
+AR = [(4, 512, 512, 64), (8, 2048, 1024, 992), (2, 2560, 768, 160), (2, 512, 256, 288)]
+AR2 = [(4, 2, 2048, 512, 96), (2, 0, 1024, 1024, 544), (8, 7, 2048, 2304, 32)]
+DONE = [(4, 512, 512, 64, False), (8, 2048, 1024, 992, False), (2, 2560, 768, 160, False), (2, 512, 256, 288, False),
+        (2, 3584, 1792, 160, False), (4, 5120, 3328, 32, False), (4, 6144, 3584, 32, False), (2, 1536, 2816, 32, False),
+        (16, 4096, 4096, 256, True), (8, 2048, 2304, 32, True), (2, 1024, 1024, 544, True), (8, 10240, 1280, 32, True)]
+
 
 def _words(n, dev):
     return torch.zeros(n, dtype=torch.int32, device=dev)
@@ -22,8 +36,7 @@ def _perm(n, dev, seed):
 
 
 @pytest.mark.parametrize("producers", [-1, -2])
-@pytest.mark.parametrize("world,M,N,K,present", [(2, 512, 256, 32, 0), (16, 4096, 256, 1056, 2), (4, 2048, 512, 992, 4),
-                                                 (8, 4096, 1024, 512, 0), (1, 256, 768, 96, 2), (3, 768, 512, 4128, 0)])
+@pytest.mark.parametrize("world,M,N,K,present", AG)
 def test_ag_small(dev, world, M, N, K, present, producers):
     print(f"ag small world={world} M={M} N={N} K={K} present={present} producers={producers}", flush=True)
     A, B = wl.randn_bf16((M, K), 1, K ** -0.5), wl.randn_bf16((K, N), 2, K ** -0.5)
@@ -48,8 +61,7 @@ def test_ag_small(dev, world, M, N, K, present, producers):
     assert torch.allclose(outs[0].cpu().float(), gemm_ref(A, B), rtol=2 ** -7, atol=1e-5)
 
 
-@pytest.mark.parametrize("world,rank,M,N,K", [(2, 1, 512, 256, 32), (16, 5, 4096, 4096, 256), (4, 0, 2048, 768, 416),
-                                              (1, 0, 512, 512, 96), (8, 7, 2048, 1024, 2080), (2, 0, 1536, 2304, 160)])
+@pytest.mark.parametrize("world,rank,M,N,K", RS)
 def test_rs_small(dev, world, rank, M, N, K):
     print(f"rs small world={world} rank={rank} M={M} N={N} K={K}", flush=True)
     A, B = wl.randn_bf16((M, K), 4, K ** -0.5), wl.randn_bf16((K, N), 5, K ** -0.5)
@@ -75,7 +87,7 @@ def test_rs_small(dev, world, rank, M, N, K):
     assert torch.allclose(outs[0][0].cpu().float(), own, rtol=2 ** -7, atol=1e-5)
 
 
-@pytest.mark.parametrize("world,M,N,K", [(4, 512, 512, 64), (8, 2048, 1024, 992), (2, 2560, 768, 160)])
+@pytest.mark.parametrize("world,M,N,K", AR)
 def test_ar_small(dev, world, M, N, K):
     print(f"ar small world={world} M={M} N={N} K={K}", flush=True)
     A, B = wl.randn_bf16((M, K), 8, K ** -0.5).to(dev), wl.randn_bf16((K, N), 9, K ** -0.5).to(dev)
@@ -96,7 +108,7 @@ def test_ar_small(dev, world, M, N, K):
     assert torch.allclose(outs[0].cpu().float(), ref, rtol=2 ** -7, atol=1e-5)
 
 
-@pytest.mark.parametrize("world,rank,M,N,K", [(4, 2, 2048, 512, 96), (2, 0, 1024, 1024, 544), (8, 7, 2048, 2304, 32)])
+@pytest.mark.parametrize("world,rank,M,N,K", AR2)
 def test_ar_two_shot_small(dev, world, rank, M, N, K):
     print(f"ar two-shot small world={world} rank={rank} M={M} N={N} K={K}", flush=True)
     A, B = wl.randn_bf16((M, K), 13, K ** -0.5).to(dev), wl.randn_bf16((K, N), 14, K ** -0.5).to(dev)
@@ -122,9 +134,7 @@ def test_ar_two_shot_small(dev, world, rank, M, N, K):
     assert int((done != 0).sum()) == s // 256 * per
 
 
-@pytest.mark.parametrize("world,M,N,K,two_shot", [(4, 512, 512, 64, False), (8, 2048, 1024, 992, False),
-                                                  (2, 2560, 768, 160, False), (16, 4096, 4096, 256, True),
-                                                  (8, 2048, 2304, 32, True), (2, 1024, 1024, 544, True)])
+@pytest.mark.parametrize("world,M,N,K,two_shot", DONE)
 def test_done_flags_come_from_the_tiles(dev, world, M, N, K, two_shot):
     """Done flags are published by the launch that folds the tiles, not by one
     behind it, under several epochs (the parts are counted in the workspace,

@@ -1,4 +1,4 @@
-"""The small-tile GEMM (problems of less than a round of 256-row tiles): edges
+"""The small-tile GEMM: edges
 of its tiles and K stages, K-split parts, strides, and what lies around the
 operands."""
 import numpy as np
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 # per tile, K of one half stage, of an odd number of half stages, and long
 SHAPES = [(128, 256, 32), (128, 256, 96), (128, 2048, 2048), (640, 512, 4128), (512, 512, 4096), (2048, 1024, 224),
           (2048, 1024, 2048), (1024, 2048, 992), (512, 2048, 8192), (2048, 2048, 1024), (1920, 2816, 608),
-          (384, 3584, 5280), (1664, 2560, 416), (4224, 2304, 288)]
+          (384, 3584, 5280), (1664, 2560, 416), (4224, 2304, 288), (512, 2816, 5984), (4480, 3584, 96),
+          (1280, 1792, 5152)]
 
 
 def _call(A, B, C, M, N, K, lda, ldb, ldc, ws):

@@ -1,0 +1,95 @@
+"""The host's choice of kernel, tile and K-split (mkernel_amd/csrc/mk_plan.h),
+compiled with the system C++ compiler: what the GPU tests' shapes are listed
+for is what they run on 256 CUs."""
+import ctypes as C
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+import test_gpu_fused_small as fused
+import test_gpu_gemm_small as small
+
+ROOT = Path(__file__).resolve().parent.parent
+
+PROG = r"""
+#include "mk_plan.h"
+static const mk::SmallSpace kSpace[2] = {{0, 0}, {496, 256LL * 262144}};
+extern "C" {
+int n_tiles() { return sizeof mk::kTiles / sizeof mk::kTiles[0]; }
+int fold_only(int i) { return mk::kTiles[i].fold_only; }
+// out: tile, workgroups, parts along K
+int gemm(int64_t M, int64_t N, int64_t K, int ws, int* out) {
+  mk::GemmSmallPlan p = {};
+  const bool s = mk::gemm_runs_small(M, N, K, K, N, 256, kSpace[ws], &p);
+  out[0] = p.tile, out[1] = p.grid, out[2] = p.split;
+  return s;
+}
+int fused(int64_t M, int64_t N, int64_t K, int peers, int64_t rows, int blocks, int second, int* out) {
+  const mk::FusedPlan f = mk::plan_fused(M, N, K, K, N, 256, {peers, rows}, blocks, second, true);
+  out[0] = f.plan.tile;
+  return f.small + 2 * f.first;
+}
+int parts(int rest, int64_t K, int bm, int n_cons, int reduce) { return mk::tail_parts(rest, K, bm, n_cons, reduce); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no host C++ compiler")
+    d = tmp_path_factory.mktemp("plans")
+    (d / "plans.cpp").write_text(PROG)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", str(ROOT / "mkernel_amd" / "csrc"),
+                    str(d / "plans.cpp"), "-o", str(d / "plans.so")], check=True, capture_output=True)
+    lib = C.CDLL(str(d / "plans.so"))
+    i64, i32 = C.c_int64, C.c_int
+    lib.gemm.argtypes = [i64, i64, i64, i32, C.c_void_p]
+    lib.fused.argtypes = [i64, i64, i64, i32, i64, i32, i32, C.c_void_p]
+    lib.parts.argtypes = [i32, i64, i32, i32, i32]
+    return lib
+
+
+def _gemm(plans, M, N, K, ws=1):
+    out = (C.c_int * 3)()
+    return bool(plans.gemm(M, N, K, ws, out)), *out
+
+
+def _fused(plans, *a):
+    out = (C.c_int * 1)()
+    f = plans.fused(*a, out)
+    return bool(f & 1), bool(f & 2), out[0]
+
+
+def test_small_gemm_shapes(plans):
+    """Each plain tile shape, and one to four parts along K, all in the small
+    kernel, with and without a workspace."""
+    got = [_gemm(plans, *s) for s in small.SHAPES]
+    assert all(g[0] for g in got) and all(_gemm(plans, *s, ws=0)[0] for s in small.SHAPES)
+    assert {g[1] for g in got} == {i for i in range(plans.n_tiles()) if not plans.fold_only(i)}
+    assert {g[3] for g in got} == {1, 2, 3, 4}
+
+
+def _blocks(world, rows, copies=1):
+    return copies * (world - 1) * rows // 128
+
+
+def test_fused_shapes(plans):
+    """Every tile shape a fold may get comes up in each operation's list, staged
+    first; the AllGather and ReduceScatter lists end in a launch that stages
+    first and then runs the persistent kernel."""
+    folds = {i for i in range(plans.n_tiles()) if 256 % (64, 128, 128, 192, 128, 128, 64)[i] == 0}
+    ag = [_fused(plans, M, N, K, -1, 0, M // 128, 0) for _, M, N, K, _ in fused.AG]
+    assert all(s and f for s, f, _ in ag[:-1]) and ag[-1][:2] == (False, True)
+    assert {t for _, _, t in ag[:-1]} == {i for i in range(plans.n_tiles()) if not plans.fold_only(i)}
+    rs = [_fused(plans, M, N, K, w - 1, M // w, _blocks(w, M // w), 0) for w, _, M, N, K in fused.RS]
+    assert all(s and f == (c[0] > 1) for (s, f, _), c in zip(rs[:-1], fused.RS)) and rs[-1][:2] == (False, True)
+    assert {t for _, _, t in rs[:-1]} == folds
+    ar = [_fused(plans, M, N, K, w - 1, M, _blocks(w, M), 0) for w, M, N, K in fused.AR]
+    ar2 = [_fused(plans, M, N, K, w - 1, M // w, _blocks(w, M // w, 2), 1) for w, _, M, N, K in fused.AR2]
+    done = [_fused(plans, M, N, K, w - 1, M // w if two else M, _blocks(w, M // w if two else M, 1 + two), two)
+            for w, M, N, K, two in fused.DONE]
+    assert all(s and f for s, f, _ in ar + ar2 + done)
+    assert {t for _, _, t in done} == folds
