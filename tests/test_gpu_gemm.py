@@ -56,9 +56,19 @@ def test_gemm_permutation_exact(dev):
     assert torch.equal(ops.gemm(P.to(dev), X.to(dev)).cpu(), X[perm])
 
 
-@pytest.mark.parametrize("M,N,K,tile,cus", [(1024, 2560, 1024, 256, 0), (768, 1024, 2048, 128, 0),
-                                             (1024, 2560, 512, 256, 96), (2048, 2048, 1024, 256, 200)])
-def test_gemm_split_tail(dev, M, N, K, tile, cus):
+def _partials(ws):
+    """Slots of 256 x 256 words that K-split parts were written to."""
+    return int((ws[4096:].view(torch.int32).view(-1, 256 * 256) != 0).any(1).sum())
+
+
+# the last: partial tiles (256 x 256 words) of tail tiles x (parts - 1)
+SPLIT_TAIL = [(1024, 2560, 4096, 256, 32, 8 * 3), (768, 1024, 2048, 128, 20, 4 * 3 // 2),
+              (1024, 2560, 4096, 256, 30, 10 * 2), (2048, 2048, 4096, 256, 48, 16 * 2),
+              (1024, 2560, 4096, 256, 0, 0)]  # a single round is not split
+
+
+@pytest.mark.parametrize("M,N,K,tile,cus,parts", SPLIT_TAIL)
+def test_gemm_split_tail(dev, M, N, K, tile, cus, parts):
     """Tail round split along K through the workspace: matches the oracle and
     the unsplit GEMM, twice in a row on one workspace (flags left zeroed)."""
     _say(f"gemm split M={M} N={N} K={K} tile={tile} cus={cus}")
@@ -75,6 +85,7 @@ def test_gemm_split_tail(dev, M, N, K, tile, cus):
         # fp32 partial sums differ from the unsplit order by fp32 rounding only
         assert torch.allclose(C.float(), plain.float(), rtol=2 ** -7, atol=1e-5)
     assert int(ws[:4096].view(torch.int32).abs().sum()) == 0, "split flags not left zeroed"
+    assert _partials(ws) == parts  # (two 128-row partial tiles fit a slot)
 
 
 @pytest.mark.parametrize("M,N,K,cus", [(8192, 3584, 256, 0),    # 448 tiles: one round + 192 spread over the XCDs
@@ -127,11 +138,12 @@ def test_gemm_random_shapes_and_grids(dev):
 
 def test_gemm_split_identity_exact(dev):
     """With a 4-way K split, I @ X is still exact (partials are exact sums)."""
-    n = 1024
-    I = torch.eye(n, dtype=torch.bfloat16, device=dev)
-    X = wl.randn_bf16((n, n), 22).to(dev)
-    assert torch.equal(ops.gemm(I, X, tile_m=256).cpu(), X.cpu())
-    assert torch.equal(ops.gemm(X, I, tile_m=128).cpu(), X.cpu())
+    for n, m, tile, cus in ((4096, 1024, 256, 60), (1024, 1024, 128, 28)):  # 4 tail tiles each
+        I = torch.eye(n, dtype=torch.bfloat16, device=dev)
+        X = wl.randn_bf16((n, m), 22).to(dev)
+        ws = torch.zeros(int(ops.capi.lib().mk_query_workspace_bytes(0, n, m, n)), dtype=torch.uint8, device=dev)
+        assert torch.equal(ops.gemm(I, X, tile_m=tile, num_cus=cus, split_ws=ws).cpu(), X.cpu())
+        assert _partials(ws) > 0
 
 
 def test_gemm_bad_shape_raises(dev):
@@ -243,8 +255,9 @@ def test_ag_gemm_epochs_and_orders(dev):
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 
 
-@pytest.mark.parametrize("num_cus,K,prod", [(4, 512, -1), (8, 1024, -1), (8, 1024, -2), (16, 512, -1), (3, 2048, -1),
-                                            (0, 512, -1), (3, 2048, -3), (8, 1024, -3), (16, 512, -6)])
+@pytest.mark.parametrize("num_cus,K,prod", [(4, 512, -1), (8, 1024, -1), (8, 1024, -2), (16, 512, -1), (3, 4096, -1),
+                                            (0, 512, -1), (3, 4096, -3), (8, 1024, -3), (16, 512, -6),
+                                            (11, 4096, -1), (5, 4096, -2)])
 def test_ag_gemm_cooperative_staging_capped_grid(dev, num_cus, K, prod):
     """Cooperative staging with a capped grid (every workgroup copies many
     pieces and computes several rounds of tiles): staged bytes and flags
@@ -252,7 +265,7 @@ def test_ag_gemm_cooperative_staging_capped_grid(dev, num_cus, K, prod):
     3 workgroups the 16 tiles leave one tail tile, split 3 ways along K while
     whole tiles follow the arrival order (a regression case: a whole tile at
     a permuted position past the split boundary once waited on the split
-    flags).  Waits are bounded so a protocol error reports instead of
+    flags); with 5 one, split 4 ways, with 11 five, split 2 ways.  Waits are bounded so a protocol error reports instead of
     hanging.  num_cus 8 and 16 (multiples of the 8 XCDs) run the schedule in
     which the two halves of the grid take turns copying ahead (-1); -2 the
     even share; -3 and -6 the co-resident staging kernel (1 and 4 staging
@@ -267,12 +280,14 @@ def test_ag_gemm_cooperative_staging_capped_grid(dev, num_cus, K, prod):
     C_ref = torch.empty((cfg.M, cfg.N), dtype=torch.bfloat16, device=dev)
     ops.ag_gemm(None, Ad, Bd, C_ref, None, None, epoch=1, gated=False, num_producers=0, num_cus=num_cus,
                 spin_limit=4_000_000, error_word=err)
+    ws = torch.zeros(int(ops.capi.lib().mk_query_workspace_bytes(0, cfg.M, cfg.N, K)), dtype=torch.uint8, device=dev)
     for epoch in (1, 2, 4):
         A_full = torch.zeros_like(Ad)
         C = torch.empty_like(C_ref)
         ops.ag_gemm(Ad, A_full, Bd, C, flags, order.to(dev), epoch=epoch, num_producers=prod, num_cus=num_cus,
-                    stage_counters=counters, spin_limit=4_000_000, error_word=err)
+                    stage_counters=counters, spin_limit=4_000_000, error_word=err, split_ws=ws)
         torch.cuda.synchronize()
+        assert _partials(ws) == {3: 2, 5: 3, 11: 5}.get(num_cus, 0)
         assert int(err.item()) == 0, "a bounded wait timed out"
         assert torch.equal(A_full.cpu(), A)
         assert (flags.cpu() == epoch).all()
@@ -308,9 +323,14 @@ def test_ag_gemm_bounded_wait_reports_timeout(dev):
 
 
 @pytest.mark.parametrize("rank,producers,num_cus,K", [(0, 4, 0, 256), (3, 8, 0, 256), (7, 0, 0, 256), (5, -1, 0, 256),
-                                                     (2, -1, 4, 1024), (6, -1, 3, 256), (1, -1, 5, 2048),
-                                                     (4, -3, 0, 256), (3, -4, 8, 512)])
+                                                     (2, -1, 4, 1024), (6, -1, 3, 256), (1, -1, 5, 14336),
+                                                     (4, -3, 0, 256), (3, -4, 8, 512), (7, -1, 5, 14336),
+                                                     (7, -1, 3, 16384), (6, -2, 11, 21504), (7, 0, 5, 14336),
+                                                     (7, -3, 5, 14336)])
 def test_gemm_rs_vs_oracle(dev, rank, producers, num_cus, K):
+    """From K 14336 on the tail of the 16 tiles is split along K, with 5
+    workgroups one tile 4 ways, with 3 one 3 ways, with 11 five 2 ways; the
+    rows of the single tail tile are rank 7's, which folds it."""
     _say(f"gemm_rs rank={rank} producers={producers} num_cus={num_cus} K={K}")
     cfg = wl.RsCfg(world=8, rank=rank, M=2048, K=K, N=512)
     A, B, peers, order = wl.rs_inputs(cfg)
@@ -326,9 +346,12 @@ def test_gemm_rs_vs_oracle(dev, rank, producers, num_cus, K):
         recv = peers.to(dev)
         flags = torch.full((nfl,), 9, dtype=torch.int32, device=dev)
     counters = torch.zeros(nfl, dtype=torch.int32, device=dev)
+    ws = torch.zeros(int(ops.capi.lib().mk_query_workspace_bytes(0, cfg.M, cfg.N, K)), dtype=torch.uint8, device=dev)
     ops.gemm_rs(Ad, Bd, work, out, peers.to(dev), recv, cfg.world, rank, flags, torch.from_numpy(order).to(dev),
-                epoch=9, num_producers=producers, stage_counters=counters, num_cus=num_cus)
+                epoch=9, num_producers=producers, stage_counters=counters, num_cus=num_cus, split_ws=ws)
     torch.cuda.synchronize()
+    assert _partials(ws) == ({3: 2, 5: 3, 11: 5}[num_cus] if K >= 14336 else 0)
+    assert int(ws[:4032].view(torch.int32).abs().sum()) == 0, "split flags not left zeroed"
     P, owned = gemm_rs_ref(A, B, peers, rank, cfg.world)
     assert rel_fro(out.float(), owned) < TOL
     mask = torch.ones(cfg.M, dtype=torch.bool)
@@ -607,13 +630,17 @@ def test_ag_gemm_cooperative_staging_full_grid_rounds(dev, prod):
     assert rel_fro(C_ref[rows].float().cpu(), gemm_ref(A[rows], B)) < TOL
 
 
-@pytest.mark.parametrize("M,N,K,cus,waves", [(2048, 1536, 2048, 32, 8),   # 48 tiles on 32: 16 split 2 ways
-                                             (2048, 1536, 2048, 40, 8),   # 8 tail tiles split 4 ways (40 // 8 > 4)
-                                             (2048, 1536, 2048, 36, 8),   # 12 tail tiles split 3 ways
-                                             (2048, 2560, 1024, 64, 8),   # 80 tiles: 16 split 4 ways
-                                             (2048, 1536, 2048, 32, 4),   # 4-wave workgroups, 2-way
-                                             (1024, 1024, 4096, 8, 8)])   # 16 tiles on 8: no tail
-def test_gemm_split_tail_exchange(dev, M, N, K, cus, waves):
+# the last: partial tiles of tail tiles x (parts - 1)
+SPLIT_EXCHANGE = [(2048, 1536, 4096, 32, 8, 16),      # 48 tiles on 32: 16 split 2 ways
+                  (2048, 1536, 4096, 40, 8, 8 * 3),   # 8 tail tiles split 4 ways (40 // 8 > 4)
+                  (2048, 1536, 4096, 36, 8, 12 * 2),  # 12 tail tiles split 3 ways
+                  (2048, 2560, 3072, 64, 8, 16 * 3),  # 80 tiles: 16 split 4 ways
+                  (2048, 1536, 4096, 32, 4, 0),       # 4-wave workgroups: never split
+                  (1024, 1024, 4096, 8, 8, 0)]        # 16 tiles on 8: no tail
+
+
+@pytest.mark.parametrize("M,N,K,cus,waves,parts", SPLIT_EXCHANGE)
+def test_gemm_split_tail_exchange(dev, M, N, K, cus, waves, parts):
     """K-split tails at capped grids: the 2-way split swaps half tiles
     between its two workgroups, wider splits fold into one owner.  Against
     the oracle, against the unsplit GEMM (fp32 rounding only), identical
@@ -630,15 +657,18 @@ def test_gemm_split_tail_exchange(dev, M, N, K, cus, waves):
     assert torch.allclose(outs[0].float(), plain.float(), rtol=2 ** -7, atol=1e-5)
     assert all(torch.equal(outs[0], o) for o in outs[1:])
     assert int(ws[:4096].view(torch.int32).abs().sum()) == 0, "split flags not left zeroed"
+    assert _partials(ws) == parts
 
 
 def test_gemm_split_tail_exchange_identity_exact(dev):
     """I @ X through a 2-way split tail is exact: each half tile's sum is the
     unsplit sum (products by 0 and 1 are exact in fp32)."""
-    n = 2048
+    n = 4096
     I = torch.eye(n, dtype=torch.bfloat16, device=dev)
-    X = wl.randn_bf16((n, 1536), 33).to(dev)
-    assert torch.equal(ops.gemm(I, X, tile_m=256, num_cus=32).cpu(), X.cpu())
+    X = wl.randn_bf16((n, 768), 33).to(dev)
+    ws = torch.zeros(int(ops.capi.lib().mk_query_workspace_bytes(0, n, 768, n)), dtype=torch.uint8, device=dev)
+    assert torch.equal(ops.gemm(I, X, tile_m=256, num_cus=32, split_ws=ws).cpu(), X.cpu())
+    assert _partials(ws) == 16
 
 
 @pytest.mark.parametrize("prod", [-1, 8, -3])

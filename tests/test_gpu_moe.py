@@ -38,8 +38,8 @@ def test_permute_bit_exact(dev):
 @pytest.mark.parametrize("split", [None, False])
 @pytest.mark.parametrize("use_rb,skip_pad", [(True, False), (False, False), (True, True)])
 def test_grouped_gemm1(dev, use_rb, skip_pad, split, tile_n):
-    """split None: the tail round is K-split through the default workspace;
-    False: no K-split."""
+    """split None: with the default workspace; False: without one (the tail
+    round is K-split from K 4096 on: test_grouped_gemm_split_tail)."""
     _say(f"moe grouped gemm1 use_rb={use_rb} skip_pad={skip_pad} split={split} tile_n={tile_n}")
     tokens, ids, gates, w1, w2, idx, d = _setup(dev)
     post = om.permute_ref(tokens, idx["pull_indices"])
@@ -380,25 +380,39 @@ def test_swiglu_epilogue_values(dev, tile_n):
     assert torch.allclose(got, ref, rtol=2 ** -7, atol=1e-30)
 
 
-def test_gemm1_swiglu_split_tail_exchange(dev):
-    """Grouped GEMM1 + SwiGLU with a capped grid so the tail round is split
-    2 ways (half-tile swap): against the oracle, bit-equal across repeated
-    launches, and within rounding of the unsplit launch."""
-    _say("moe gemm1+swiglu split exchange")
-    tokens, ids, gates, w1, w2, idx, d = _setup(dev, WIDE)
+DEEP = wl.MoeCfg(tokens=512, H=4128, I=512, experts=64, topk=8, ep=8, rank=1)
+
+
+@pytest.mark.parametrize("mode,tile_n", [(1, 512), (0, 512), (1, 256)])
+@pytest.mark.parametrize("parts", [2, 3, 4])
+@pytest.mark.parametrize("sized", [False, True])
+def test_grouped_gemm_split_tail(dev, mode, tile_n, parts, sized):
+    """Expert GEMMs with a capped grid so that the tail round is split 2 ways
+    (half-tile swap), 3 or 4 ways (one owner), planned on the host or, with a
+    device row count, in the kernel: against the oracle, bit-equal across
+    repeated launches, and within rounding of the unsplit launch."""
+    tokens, ids, gates, w1, w2, idx, d = _setup(dev, DEEP)
     post = om.permute_ref(tokens, idx["pull_indices"])
-    ntiles = (idx["R_pad"] // 128) * (2 * WIDE.I // 512)
-    # a grid whose tail (ntiles % cus tiles) the library splits 2 ways: cus / tail in [2, 3)
-    cus = next(c for c in range(2, ntiles) if ntiles % c and 2 <= c // (ntiles % c) < 3)
+    R_pad, width = idx["R_pad"], 2 * DEEP.I
+    ntiles = (R_pad // 128) * (width // tile_n)
+    # the smallest grid whose tail (ntiles % cus tiles) is split `parts` ways
+    cus = next(c for c in range(2, ntiles) if ntiles % c and min(4, c // (ntiles % c)) == parts)
+    _say(f"moe split tail mode={mode} tile_n={tile_n} parts={parts} sized={sized} tiles={ntiles} cus={cus}")
+    sizes = torch.tensor([idx["R"], R_pad], dtype=torch.int64, device=dev) if sized else None
+    ws = torch.zeros(int(ops.capi.lib().mk_query_workspace_bytes(0, 0, 0, 0)), dtype=torch.uint8, device=dev)
     outs = []
-    for split in (None, None, False):
-        act = torch.empty((idx["R_pad"], WIDE.I), dtype=torch.bfloat16, device=dev)
-        ops.moe_grouped_gemm(post.to(dev), w1.to(dev), act, rb_expert=d["rb_expert"], mode=1, split_ws=split,
-                             tile_n=512, num_cus=cus)
+    for split in (ws, ws, False):
+        act = torch.empty((R_pad, width // (1 + mode)), dtype=torch.bfloat16, device=dev)
+        ops.moe_grouped_gemm(post.to(dev), w1.to(dev), act, rb_expert=d["rb_expert"], mode=mode, split_ws=split,
+                             tile_n=tile_n, num_cus=cus, sizes=sizes)
         outs.append(act)
     torch.cuda.synchronize()
-    ref_act, _ = om.ffn_ref(post, w1, w2, idx["padded_tokens_per_expert"], WIDE.I)
-    assert rel_fro(outs[0].float().cpu(), ref_act) < TOL
+    written = int((ws[4096:].view(torch.int32).view(-1, 128 * tile_n) != 0).any(1).sum())
+    assert written == ntiles % cus * (parts - 1)
+    assert not bool(ws[:4096].any()), "split flags not left zeroed"
+    ref = (om.ffn_ref(post, w1, w2, idx["padded_tokens_per_expert"], DEEP.I)[0] if mode
+           else om.grouped_gemm_ref(post, w1, idx["padded_tokens_per_expert"]))
+    assert rel_fro(outs[0].float().cpu(), ref) < TOL
     assert torch.equal(outs[0], outs[1])
     assert torch.allclose(outs[0].float(), outs[2].float(), rtol=2 ** -6, atol=1e-3)
 

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from mkernel_amd import ops, workloads as wl
+from mkernel_amd import capi, ops, workloads as wl
 
 pytestmark = pytest.mark.gpu
 
@@ -101,6 +101,8 @@ def test_index_dev_feeds_ffn(dev):
 LAYER = wl.MoeCfg(tokens=512, H=512, I=256, experts=64, topk=8, ep=8, rank=0)
 # GEMM2 with 9 column tiles of 512 (more than 8: the expert tile order)
 LAYER_WIDE = wl.MoeCfg(tokens=512, H=4608, I=256, experts=64, topk=8, ep=8, rank=0)
+# GEMM1 with a K that is split in the tail round
+LAYER_DEEP = wl.MoeCfg(tokens=512, H=4352, I=256, experts=64, topk=8, ep=8, rank=0)
 
 
 def _host_layer(dev, cfg, tokens, w1, w2, ids, gates, split_ws, fuse):
@@ -152,9 +154,8 @@ def _routing(cfg, seed):
 def test_layer_with_device_row_count(dev, fuse, wide):
     """Without the K-split every output tile is one workgroup's full-K sum,
     so the capacity-sized launch gives the host-sized launch's bits; with the
-    split (planned on the device) it stays within the parity bound.  wide:
-    GEMM2 has more than 8 column tiles, so both launches walk the tiles in
-    expert order, the device one over its clamped row tiles."""
+    split (planned on the device; wide: GEMM1's K is long enough for it) it
+    stays within the parity bound.  wide: GEMM2 has more than 8 column tiles."""
     _say(f"moe layer, device row count, fuse={fuse} wide={wide}")
     from oracle.gemm import rel_fro
     cfg = LAYER_WIDE if wide else LAYER
@@ -180,11 +181,13 @@ def test_layer_graph_replays(dev, split):
     eager run on the same routing (bit-exact), with eager library work and
     synchronizations between the replays."""
     _say(f"moe layer graph replays split={split}")
-    cfg = LAYER
+    cfg = LAYER if split is False else LAYER_DEEP
     tokens, _, _, w1, w2 = wl.moe_inputs(cfg)
     tokens, w1, w2 = tokens.to(dev), w1.to(dev), w2.to(dev)
     ids0, gates0 = _routing(cfg, 6)
     ids_d, gates_d = torch.from_numpy(ids0).to(dev), torch.from_numpy(gates0).to(dev)
+    if split is None:
+        split = torch.zeros(int(capi.lib().mk_query_workspace_bytes(0, 0, 0, 0)), dtype=torch.uint8, device=dev)
     layer = _DeviceLayer(dev, cfg, tokens, w1, w2, ids_d, gates_d, split, False)
     eager = {}
     for seed in (6, 7, 8):
@@ -199,9 +202,12 @@ def test_layer_graph_replays(dev, split):
         ids, gates = _routing(cfg, seed)
         ids_d.copy_(torch.from_numpy(ids)); gates_d.copy_(torch.from_numpy(gates))
         layer.y.fill_(-1.0)
+        if split is not False:
+            split[4096:].zero_()
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(layer.y, eager[seed]), seed
+        assert split is False or (bool(split[4096:].any()) and not bool(split[:4096].any()))
         # eager library work between replays
         ops.gemm(tokens[:256], w1[0, :, :256].contiguous())
         torch.cuda.synchronize()

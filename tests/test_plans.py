@@ -9,7 +9,9 @@ from pathlib import Path
 import pytest
 
 import test_gpu_fused_small as fused
+import test_gpu_gemm as dense
 import test_gpu_gemm_small as small
+import test_zz_no_alloc as noalloc
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -93,3 +95,26 @@ def test_fused_shapes(plans):
             for w, M, N, K, two in fused.DONE]
     assert all(s and f for s, f, _ in ar + ar2 + done)
     assert {t for _, _, t in done} == folds
+
+
+def test_split_tail_shapes(plans):
+    """The dense K-split tests' tail tiles are split as their lists say, with
+    two, three and four parts among them."""
+    seen = set()
+
+    def partials(tiles, K, bm, cus, reduce=0):
+        cus = min(cus, tiles)  # the grid
+        rest = tiles % cus
+        s = plans.parts(rest, K, bm, cus, reduce)
+        seen.add(s)
+        return rest * (s - 1) * bm // 256
+
+    for M, N, K, bm, cus, want in dense.SPLIT_TAIL:
+        assert partials((M // bm) * (N // 256), K, bm, cus or 256) == want
+    for M, N, K, cus, waves, want in dense.SPLIT_EXCHANGE:
+        assert want == (0 if waves == 4 else partials((M // 256) * (N // 256), K, 256, cus))
+    for world, rows, K, N, want in noalloc.NOALLOC_SPLIT:
+        assert partials(world * rows // 256 * (N // 256), K, 256, 256) == want
+    assert seen >= {2, 3, 4}
+    # with the fold, 16 tiles on 5, 3 and 11 workgroups
+    assert [plans.parts(16 % c, K, 256, c, 1) for c, K in ((5, 14336), (3, 16384), (11, 21504), (5, 4096))] == [4, 3, 2, 1]
