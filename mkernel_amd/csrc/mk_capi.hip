@@ -165,6 +165,7 @@ mk::GemmSmallParams small_params(const mk::GemmSmallPlan& plan, const void* A, c
   p.tiles_n = (int)(N / plan.bn);
   p.group_m = 8;
   p.nk = (int)((K + 63) / 64);
+  p.split = plan.split;
   return p;
 }
 

@@ -1,14 +1,12 @@
-// mk_gemm_small.hip — bf16 GEMM for problems of less than one round of the
-// persistent kernel's tiles (gfx950).
+// mk_gemm_small.hip — bf16 GEMM on tiles of 64 x 64 to 128 x 256 (gfx950): for
+// problems that leave the chip idle at the persistent kernel's tiles, and for
+// those of any size that cost less in rounds of these (mk_plan.h).
 //
 // The persistent kernel runs 128 x 256 or 256 x 256 tiles, one workgroup per
 // CU; a 128 x 2048 x 2048 product is eight such tiles, so eight of 256 CUs
 // work and each streams a whole K panel alone.  Here the tile is chosen to
-// fill the chip (64 x 64 .. 128 x 256) and, where even that leaves CUs idle,
-// the K stages of all tiles are dealt out evenly over the workgroups:
-// workgroup w takes the stages [w, w + 1) * total / G of the tile-major
-// stage sequence, so it holds at most one part of a tile at either end and
-// whole tiles between.
+// fill the chip and, where even that leaves CUs idle, each tile's K is cut
+// into two to four parts, a workgroup each.
 //
 // Parts of one tile meet in the workspace.  Every part takes a ticket when
 // its sum is done; all but the last write their fp32 sums there and publish a
@@ -49,6 +47,10 @@ struct SCfg {
   static constexpr int B_UPR = BN / 8;  // 16-byte units per B k-row
   static constexpr uint32_t STAGE = A_BYTES + BK * BROW;
   static constexpr uint32_t LDS_BYTES = S * STAGE;
+  // what the ring lets run: the compiler, which cannot know a launch's LDS,
+  // else saves registers for more waves and serialises the LDS reads of a stage
+  // (128x2048x2048 11.0 us so, 10.0 with the limit)
+  static constexpr int WAVES_PER_SIMD = 160 * 1024 / LDS_BYTES * WAVES / 4;
   static constexpr int A_INST = A_BYTES / 1024 / WAVES;
   static constexpr int B_INST = BK * BROW / 1024 / WAVES;
   static constexpr int LOADS = A_INST + B_INST;
@@ -144,7 +146,7 @@ __device__ __forceinline__ void part_done(const GemmSmallParams& p, int row, int
 }
 
 template <class C, bool REDUCE>
-__global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p) {
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(1, C::WAVES_PER_SIMD))) void gemm_small_kernel(GemmSmallParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / C::WN, wn = wave % C::WN;
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
   // has one id more than G / 8 while x < G % 8)
   const uint32_t G = gridDim.x, xcd = blockIdx.x & 7;
   const uint32_t id = xcd * (G >> 3) + min(xcd, G & 7) + (blockIdx.x >> 3);
-  const uint32_t nk = p.nk, total = p.tiles_m * p.tiles_n * nk;
+  const uint32_t t = REDUCE ? id : id / p.split, part = REDUCE ? 0 : id - t * p.split;  // a fold's tiles are whole
 
   const int ml = lane & 31, g = lane >> 5;
   uint32_t a_rd[4];
@@ -186,148 +188,138 @@ __global__ __launch_bounds__(C::NT, 1) void gemm_small_kernel(GemmSmallParams p)
     b_chk[i] = (n % C::B_UPR) ^ b_swizzle<C::BN>(b_row[i]);
   }
 
-  uint32_t st = (uint32_t)((uint64_t)id * total / G);
-  const uint32_t end = (uint32_t)((uint64_t)(id + 1) * total / G);
-  while (st < end) {
-    const uint32_t t = st / nk, k0 = st - t * nk;
-    const int n = (int)min(nk - k0, end - st);
-    st += n;
-    int tm, tn;
-    decode_grouped((int)t, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
-    // The rows to fold cost more than the others and are neighbours: each
-    // eighth of the columns starts its walk over the rows another eighth
-    // further on, so that the fold falls on every XCD.
-    if (REDUCE) tm = (tm + tn * 8 / p.tiles_n * ((p.tiles_m + 7) / 8)) % p.tiles_m;
-    const int m0 = __builtin_amdgcn_readfirstlane(tm * C::BM), n0 = __builtin_amdgcn_readfirstlane(tn * C::BN);
-    const u32x4_t rA = make_rsrc_v(p.A + (int64_t)m0 * p.lda, (uint32_t)(C::BM * p.lda * 2));
-    const u32x4_t rB = make_rsrc_v(p.B, (uint32_t)(p.K * p.ldb * 2));
-    uint32_t a_src[C::A_INST], b_src[C::B_INST];
+  const uint32_t k0 = REDUCE ? 0 : part * p.nk / p.split;
+  const int n = (REDUCE ? p.nk : (int)((part + 1) * p.nk / p.split)) - (int)k0;
+  int tm, tn;
+  decode_grouped((int)t, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
+  // The rows to fold cost more than the others and are neighbours: each
+  // eighth of the columns starts its walk over the rows another eighth
+  // further on, so that the fold falls on every XCD.
+  if (REDUCE) tm = (tm + tn * 8 / p.tiles_n * ((p.tiles_m + 7) / 8)) % p.tiles_m;
+  const int m0 = __builtin_amdgcn_readfirstlane(tm * C::BM), n0 = __builtin_amdgcn_readfirstlane(tn * C::BN);
+  const u32x4_t rA = make_rsrc_v(p.A + (int64_t)m0 * p.lda, (uint32_t)(C::BM * p.lda * 2));
+  const u32x4_t rB = make_rsrc_v(p.B, (uint32_t)(p.K * p.ldb * 2));
+  uint32_t a_src[C::A_INST], b_src[C::B_INST];
 #pragma unroll
-    for (int i = 0; i < C::A_INST; ++i) a_src[i] = (uint32_t)(a_row[i] * p.lda * 2 + a_chk[i] * 16);
+  for (int i = 0; i < C::A_INST; ++i) a_src[i] = (uint32_t)(a_row[i] * p.lda * 2 + a_chk[i] * 16);
 #pragma unroll
-    for (int i = 0; i < C::B_INST; ++i) b_src[i] = (uint32_t)(b_row[i] * p.ldb * 2 + (n0 + b_chk[i] * 8) * 2);
-    // ring slots as byte offsets, stepped (a modulo of the stage number costs
-    // more than a DMA's issue when S is not a power of two)
-    auto next_slot = [](uint32_t o) { return o + C::STAGE == C::LDS_BYTES ? 0u : o + C::STAGE; };
-    uint32_t wr = 0, rd = 0;
-    uint32_t ka = k0 * (C::BK * 2), kb = k0 * (uint32_t)(C::BK * p.ldb * 2);
-    // a tile whose K holds an odd number of 32-deep steps ends in a half stage
-    int half = (p.K & 32) ? (int)(nk - 1 - k0) : -1;
-    auto issue = [&] {
-      const uint32_t slot = lds_base + wr;
-      if (half == 0) {
-        // the half stage: its second 32 K steps read as zeros (offsets past
-        // both buffers' ends)
-        uint32_t av[C::A_INST], bv[C::B_INST];
+  for (int i = 0; i < C::B_INST; ++i) b_src[i] = (uint32_t)(b_row[i] * p.ldb * 2 + (n0 + b_chk[i] * 8) * 2);
+  // ring slots as byte offsets, stepped (a modulo of the stage number costs
+  // more than a DMA's issue when S is not a power of two)
+  auto next_slot = [](uint32_t o) { return o + C::STAGE == C::LDS_BYTES ? 0u : o + C::STAGE; };
+  uint32_t wr = 0, rd = 0;
+  uint32_t ka = k0 * (C::BK * 2), kb = k0 * (uint32_t)(C::BK * p.ldb * 2);
+  // a tile whose K holds an odd number of 32-deep steps ends in a half stage
+  int half = (p.K & 32) ? p.nk - 1 - (int)k0 : -1;
+  auto issue = [&] {
+    const uint32_t slot = lds_base + wr;
+    if (half == 0) {
+      // the half stage: its second 32 K steps read as zeros (offsets past
+      // both buffers' ends)
+      uint32_t av[C::A_INST], bv[C::B_INST];
 #pragma unroll
-        for (int i = 0; i < C::A_INST; ++i) av[i] = a_chk[i] < 4 ? a_src[i] : 0x80000000u;
+      for (int i = 0; i < C::A_INST; ++i) av[i] = a_chk[i] < 4 ? a_src[i] : 0x80000000u;
 #pragma unroll
-        for (int i = 0; i < C::B_INST; ++i) bv[i] = b_row[i] < 32 ? b_src[i] : 0x80000000u;
-        dma16_run<C::A_INST>(rA, slot + wave_u * C::A_INST * 1024, av, ka);
-        dma16_run<C::B_INST>(rB, slot + C::A_BYTES + wave_u * C::B_INST * 1024, bv, kb);
-      } else {
-        dma16_run<C::A_INST>(rA, slot + wave_u * C::A_INST * 1024, a_src, ka);
-        dma16_run<C::B_INST>(rB, slot + C::A_BYTES + wave_u * C::B_INST * 1024, b_src, kb);
+      for (int i = 0; i < C::B_INST; ++i) bv[i] = b_row[i] < 32 ? b_src[i] : 0x80000000u;
+      dma16_run<C::A_INST>(rA, slot + wave_u * C::A_INST * 1024, av, ka);
+      dma16_run<C::B_INST>(rB, slot + C::A_BYTES + wave_u * C::B_INST * 1024, bv, kb);
+    } else {
+      dma16_run<C::A_INST>(rA, slot + wave_u * C::A_INST * 1024, a_src, ka);
+      dma16_run<C::B_INST>(rB, slot + C::A_BYTES + wave_u * C::B_INST * 1024, b_src, kb);
+    }
+    --half;
+    ka += C::BK * 2;
+    kb += (uint32_t)(C::BK * p.ldb * 2);
+    wr = next_slot(wr);
+  };
+  f32x16 acc[C::FM][C::FN];
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  auto compute = [&] {
+    const char* sA = smem + rd;
+    const char* sB = sA + C::A_BYTES;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      bf16x8 af[C::FM], bf[C::FN];
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(sA + a_rd[kk] + i * 32 * 128);
+#pragma unroll
+      for (int jj = 0; jj < C::FN; ++jj) {
+        const bf16x4_t lo = lds_tr4(sB + b_rd[jj] + kk * 16 * C::BROW);
+        const bf16x4_t hi = lds_tr4(sB + b_rd[jj] + kk * 16 * C::BROW + 4 * C::BROW);
+        bf[jj] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       }
-      --half;
-      ka += C::BK * 2;
-      kb += (uint32_t)(C::BK * p.ldb * 2);
-      wr = next_slot(wr);
-    };
-    f32x16 acc[C::FM][C::FN];
 #pragma unroll
-    for (int i = 0; i < C::FM; ++i)
+      for (int i = 0; i < C::FM; ++i)
 #pragma unroll
-      for (int j = 0; j < C::FN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    auto compute = [&] {
-      const char* sA = smem + rd;
-      const char* sB = sA + C::A_BYTES;
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        bf16x8 af[C::FM], bf[C::FN];
-#pragma unroll
-        for (int i = 0; i < C::FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(sA + a_rd[kk] + i * 32 * 128);
-#pragma unroll
-        for (int jj = 0; jj < C::FN; ++jj) {
-          const bf16x4_t lo = lds_tr4(sB + b_rd[jj] + kk * 16 * C::BROW);
-          const bf16x4_t hi = lds_tr4(sB + b_rd[jj] + kk * 16 * C::BROW + 4 * C::BROW);
-          bf[jj] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-#pragma unroll
-        for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-          for (int jj = 0; jj < C::FN; ++jj)
-            acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[jj], af[i], acc[i][jj], 0, 0, 0);
-      }
-      rd = next_slot(rd);
-    };
+        for (int jj = 0; jj < C::FN; ++jj)
+          acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[jj], af[i], acc[i][jj], 0, 0, 0);
+    }
+    rd = next_slot(rd);
+  };
 
 #pragma unroll
-    for (int s = 0; s < C::S - 1; ++s)
-      if (s < n) issue();
-    // Each barrier says that every wave's share of stage j has landed and that
-    // every wave has read stage j - 1, whose slot the next DMA overwrites.
-    int j = 0;
-    for (; j + C::S - 1 < n; ++j) {
-      wait_vm<(C::S - 2) * C::LOADS>();
+  for (int s = 0; s < C::S - 1; ++s)
+    if (s < n) issue();
+  // Each barrier says that every wave's share of stage j has landed and that
+  // every wave has read stage j - 1, whose slot the next DMA overwrites.
+  int j = 0;
+  for (; j + C::S - 1 < n; ++j) {
+    wait_vm<(C::S - 2) * C::LOADS>();
+    __syncthreads();
+    issue();
+    compute();
+  }
+  for (; j < n; ++j) {
+    wait_pending<C::S - 2, C::LOADS>(n - 1 - j);
+    __syncthreads();
+    compute();
+  }
+  __syncthreads();  // the ring is free: the exchange and the store use it
+  if (!REDUCE && p.split > 1) {
+    const int parts = p.split, w0 = (int)t * parts;  // the tile's first workgroup, whose slots its parts use
+    int* sh = reinterpret_cast<int*>(smem);
+    uint32_t* ticket = p.words + t;
+    uint32_t* head = p.words + p.tiles_m * p.tiles_n + w0;  // one per part but the last
+    if (tid == 0) sh[0] = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int tk = __builtin_amdgcn_readfirstlane(sh[0]);
+    float* slot0 = p.ws + (int64_t)w0 * (C::BM * C::BN);
+    if (tk < parts - 1) {
+      part_out<C>(slot0 + (int64_t)tk * (C::BM * C::BN), acc, tid);
+      // write-through stores performed at agent scope, then a relaxed flag
+      wait_vmem_all();
       __syncthreads();
-      issue();
-      compute();
+      if (tid == 0)
+        __hip_atomic_store(head + tk, part + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
     }
-    for (; j < n; ++j) {
-      wait_pending<C::S - 2, C::LOADS>(n - 1 - j);
-      __syncthreads();
-      compute();
+    if (tid < parts - 1) {
+      uint32_t h;
+      while ((h = __hip_atomic_load(head + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0u)
+        __builtin_amdgcn_s_sleep(1);
+      sh[1 + (h - 1u)] = tid;
+      // every part is in: both words are clear for the next launch
+      __hip_atomic_store(head + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __syncthreads();  // the ring is free: the exchange and the store use it
-    if (!REDUCE && n < (int)nk) {
-      // first and last workgroup with a part of this tile
-      const uint32_t f0 = t * nk, f1 = f0 + nk - 1;
-      const uint32_t w0 = (uint32_t)(((uint64_t)(f0 + 1) * G - 1) / total);
-      const uint32_t w1 = (uint32_t)(((uint64_t)(f1 + 1) * G - 1) / total);
-      const int parts = (int)(w1 - w0) + 1, own = (int)(id - w0);
-      int* sh = reinterpret_cast<int*>(smem);
-      uint32_t* ticket = p.words + t;
-      uint32_t* head = p.words + p.tiles_m * p.tiles_n + w0;  // one per part but the last
-      if (tid == 0) sh[0] = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      const int tk = __builtin_amdgcn_readfirstlane(sh[0]);
-      float* slot0 = p.ws + (int64_t)w0 * (C::BM * C::BN);
-      if (tk < parts - 1) {
-        part_out<C>(slot0 + (int64_t)tk * (C::BM * C::BN), acc, tid);
-        // write-through stores performed at agent scope, then a relaxed flag
-        wait_vmem_all();
-        __syncthreads();
-        if (tid == 0)
-          __hip_atomic_store(head + tk, (uint32_t)own + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        continue;
-      }
-      if (tid < parts - 1) {
-        uint32_t h;
-        while ((h = __hip_atomic_load(head + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0u)
-          __builtin_amdgcn_s_sleep(1);
-        sh[1 + (h - 1u)] = tid;
-        // every part is in: both words are clear for the next launch
-        __hip_atomic_store(head + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      __syncthreads();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      parts_in<C>(slot0, sh + 1, parts, own, acc, tid);
-      __syncthreads();  // sh is read: the store reuses the LDS
-    }
-    if (REDUCE && m0 >= p.rs_own_row0 && m0 < p.rs_own_row0 + p.rs_own_rows) {
-      static_assert(!REDUCE || C::WAVES * 32 * (C::WTN * 4 + 16) <= C::LDS_BYTES, "fold rows in LDS");
-      reduce_rows<C, 8, true>(p, acc, m0 - p.rs_own_row0 + wm * C::WTM, n0 + wn * C::WTN, smem, wave, lane);
-      if (p.done) part_done<C>(p, m0 - p.rs_own_row0, n0, tid);
-    } else {
-      // with the fold these are the would-be sends: written once, not read here
-      store_rows<C, C::FN, REDUCE>(p.C + (int64_t)(m0 + wm * C::WTM) * p.ldc + n0 + wn * C::WTN, p.ldc, acc, smem, wave,
-                                   lane);
-    }
-    if (st < end) __syncthreads();  // the ring is refilled by the next tile
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    parts_in<C>(slot0, sh + 1, parts, (int)part, acc, tid);
+    __syncthreads();  // sh is read: the store reuses the LDS
+  }
+  if (REDUCE && m0 >= p.rs_own_row0 && m0 < p.rs_own_row0 + p.rs_own_rows) {
+    static_assert(!REDUCE || C::WAVES * 32 * (C::WTN * 4 + 16) <= C::LDS_BYTES, "fold rows in LDS");
+    reduce_rows<C, 8, true>(p, acc, m0 - p.rs_own_row0 + wm * C::WTM, n0 + wn * C::WTN, smem, wave, lane);
+    if (p.done) part_done<C>(p, m0 - p.rs_own_row0, n0, tid);
+  } else {
+    // with the fold these are the would-be sends: written once, not read here
+    store_rows<C, C::FN, REDUCE>(p.C + (int64_t)(m0 + wm * C::WTM) * p.ldc + n0 + wn * C::WTN, p.ldc, acc, smem, wave,
+                                 lane);
   }
 }
 

@@ -121,6 +121,7 @@ struct GemmSmallParams {
   int K;
   int tiles_m, tiles_n, group_m;
   int nk;            // 64-deep K stages of a tile
+  int split;         // parts of a tile along K (1: whole)
   // zero between launches: a ticket per tile and a header per workgroup of a
   // K-split; with done flags, the finished parts of each
   uint32_t* words;
