@@ -182,15 +182,18 @@ inline bool gemm_runs_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_
   const bool split = ws.words > 0;
   const int64_t t256 = M % 256 ? 0 : (M / 256) * (N / 256);
   if (2 * t256 > cus && persistent_cost(t256, K, cus, split) <= plan->us) return false;
-  // An odd number of 128-row blocks, a little over one round of 128 x 256 tiles
-  // and a long K: the persistent kernel splits the few tiles of the second
-  // round.  us, its time against two rounds of small tiles: K 4096 within 4 % of
-  // each other at 260 to 318 tiles of 512 to 2048 columns; K 5504 120 / 122 (264
-  // tiles), 121 / 130 (296), 124 / 123 (312); K 8192 169 / 178, 172 / 184, 174 /
-  // 181; K 14336 284 / 306, 289 / 324, 292 / 316; 256 columns, 289 tiles: K 4096
-  // 103 / 126, K 14336 331 / 526.  At K 3072, 261 tiles: 77 / 75.
-  const int64_t t128 = (M / 128) * (N / 256);
-  return !(M % 256 && split && K >= 4096 && t128 > cus && 4 * t128 <= 5 * cus);
+  // An odd number of 128-row blocks, a last round of 128 x 256 tiles that can be
+  // split along K, and a K long enough for it (the more rounds, the less the
+  // last one weighs): the persistent kernel.  us, its time against the small
+  // tiles': 264 tiles K 4096 104 / 102, 5504 120 / 122, 14336 284 / 306; 289 of
+  // 256 columns 4096 103 / 126, 14336 331 / 526; 345 K 4384 112 / 117, 13472 336 /
+  // 478; 536 K 15072 551 / 673; 595 K 4928 216 / 189, 10656 432 / 546; 820 K 5408
+  // 306 / 342; 1050 K 4832 356 / 344; 1090 K 13856 1011 / 1115.  A fuller last
+  // round gains nothing (418 tiles K 10016 333 / 330, 472 K 14688 483 / 442).
+  // Over 267 such shapes the choice costs 0.7 % in the mean, 2.2 % when the line
+  // was at 320 tiles of K 4096 and more.
+  const int64_t t128 = (M / 128) * (N / 256), rounds = t128 / cus, rest = t128 % cus;
+  return !(M % 256 && split && rounds && rest && 20 * rest <= 9 * cus && K >= 1000 * (rounds + 3));
 }
 
 struct FusedPlan {

@@ -671,6 +671,28 @@ def test_gemm_split_tail_exchange_identity_exact(dev):
     assert _partials(ws) == 16
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(4224, 2048, 4096, 8 * 3), (8320, 2048, 5024, 8 * 3),
+                                         (13952, 768, 5024, 71 * 2)])
+def test_gemm_odd_row_blocks_split_tail(dev, M, N, K, parts):
+    """128-row tiles in one and two whole rounds of 256 workgroups and a last
+    round split along K (8 tiles four ways, 8 four ways, 71 three ways), chosen
+    by the library: against the oracle in the first and last rows, against
+    whole tiles everywhere."""
+    if ops.cu_count() != 256:
+        pytest.skip("rounds are for 256 CUs")
+    _say(f"gemm odd row blocks M={M} N={N} K={K}")
+    A = wl.randn_bf16((M, K), 34, K ** -0.5)
+    B = wl.randn_bf16((K, N), 35, K ** -0.5)
+    ws = torch.zeros(int(ops.capi.lib().mk_query_workspace_bytes(0, M, N, K)), dtype=torch.uint8, device=dev)
+    outs = [ops.gemm(A.to(dev), B.to(dev), split_ws=w) for w in (ws, ws, False)]
+    torch.cuda.synchronize()
+    assert int((ws[4096:].view(torch.int32).view(-1, 128 * 256) != 0).any(1).sum()) == parts
+    assert not bool(ws[:4096].any()) and torch.equal(outs[0], outs[1])
+    assert torch.allclose(outs[0].float(), outs[2].float(), rtol=2 ** -7, atol=1e-5)
+    for rows in (slice(0, 256), slice(M - 384, M)):
+        assert torch.allclose(outs[0][rows].cpu().float(), gemm_ref(A[rows], B), rtol=2 ** -7, atol=1e-5)
+
+
 @pytest.mark.parametrize("prod", [-1, 8, -3])
 def test_ag_gemm_graph_replays_device_epoch(dev, prod):
     """AllGather+GEMM recorded once in a HIP graph after mk_epoch_advance,

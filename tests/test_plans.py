@@ -74,6 +74,17 @@ def test_small_gemm_shapes(plans):
     assert {g[3] for g in got} == {1, 2, 3, 4}
 
 
+@pytest.mark.parametrize("M,N,K,persistent", [(4224, 2048, 5504, 1), (36992, 256, 4096, 1), (4224, 2048, 3072, 0),
+                                              (14720, 768, 13472, 1), (8320, 2048, 5024, 1), (22400, 768, 9056, 1),
+                                              (15232, 1280, 4928, 0), (26240, 1024, 7712, 1), (22400, 1536, 4832, 0),
+                                              (26752, 512, 10016, 0), (16512, 1024, 8192, 1), (32640, 512, 8192, 0)])
+def test_odd_row_blocks(plans, M, N, K, persistent):
+    """Odd numbers of 128-row blocks go to the persistent kernel where its last
+    round is split along K and K is long for the number of rounds; without a
+    workspace there is no split."""
+    assert _gemm(plans, M, N, K)[0] != bool(persistent) and _gemm(plans, M, N, K, ws=0)[0]
+
+
 def _blocks(world, rows, copies=1):
     return copies * (world - 1) * rows // 128
 
