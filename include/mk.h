@@ -46,12 +46,14 @@ typedef struct mk_gemm_args {
   int64_t M, N, K;
   int64_t lda, ldb, ldc;
   int32_t num_cus; /* persistent grid size; 0 = every CU of the device; at most the CU count */
-  int32_t tile_m;  /* 0 = auto (256 unless 128-row tiles fit in one round
-                      of the grid), else 128 or 256 */
+  int32_t tile_m;  /* 0 = auto; 128 or 256: the persistent kernel's tile height.  With
+                      tile_m, waves and num_cus all 0 the library chooses between that
+                      kernel and one on tiles of 64 x 64 to 128 x 256 */
   int32_t waves;   /* waves per workgroup: 0 = auto, 4 (one per SIMD) or 8 (two per SIMD) */
   void* split_ws;          /* optional K-split workspace (see mk_query_workspace_bytes);
                               zero-filled before its first use, left zeroed by every
-                              launch; NULL = no K-split of the tail round */
+                              launch; NULL = no tile is split along K (neither the
+                              tail round's nor a small problem's) */
   int64_t split_ws_bytes;
 } mk_gemm_args;
 int mk_gemm(const mk_gemm_args* args, void* stream);
@@ -204,7 +206,8 @@ int mk_gemm_rs(const mk_gemm_rs_args* args, void* stream);
  * row tile's last peer block.  When done_flags is set, each finished
  * 256x256 output tile t = row_tile * (N/256) + col_tile is published as
  * done_flags[t] = epoch after its bytes are visible at agent scope (the hand-off
- * the reference's broadcast step reads).
+ * the reference's broadcast step reads); a copy kernel that stages first
+ * (num_producers -1 or -2) delays the first of them by its own time.
  * Replaces gemm_ar_multinode::entrypoint
  * (reference include/operators/gemm_ar/session.cuh:188-215,
  * src/gemm_ar.cu:1-33 compute + intra-AR roles; the reference checks

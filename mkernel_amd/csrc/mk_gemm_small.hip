@@ -25,8 +25,8 @@
 // Bound by latency below ~1 GFLOP and by the operand stream through L2 / LDS
 // above (a 128 x 128 tile moves 64 bytes per MFMA cycle).  Measured against
 // the persistent kernel's 128 x 256 tiles on one MI355X (us): 128x2048x2048
-// 31.9 -> 10.9, 1024^3 18.7 -> 6.8, 512x2048x8192 112 -> 31, 2048^3 33 -> 22,
-// 2048x2048x8192 115 -> 76, 1920x2816x5600 79.5 -> 71.2.
+// 31.9 -> 10.0, 1024^3 18.7 -> 6.8, 512x2048x8192 112 -> 31, 2048^3 33 -> 22,
+// 2048x2048x8192 115 -> 76, 1920x2816x5600 79.5 -> 69.
 #include "mk_device.h"
 #include "mk_internal.h"
 #include "mk_once.h"

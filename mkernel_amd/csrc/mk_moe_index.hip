@@ -23,7 +23,7 @@
 //   scatter per chunk: stable rank within the chunk, row, slot -> routed rows
 //           per 256 rows < R_pad: expert of the row, padding rows, row-block tables
 // (plan leaves the chunk prefixes relative to the expert and scatter adds the
-// expert's offset: rewriting them took 3 of plan's 30 us at 16384 tokens.)
+// expert's offset: rewriting them took 2.4 of plan's 27 us at 16384 tokens.)
 //
 // A small batch (a decode step: at most kSmallEntries entries, kSmallThreads
 // tokens and kSmallExperts experts) is one workgroup's work and one launch
