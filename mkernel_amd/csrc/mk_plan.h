@@ -170,6 +170,13 @@ inline int tail_parts(int R, int64_t K, int bm, int n_cons, bool reduce) {
   return (int)std::min<int64_t>(std::min(4, n_cons / R), (K / 32) / 4);
 }
 
+// The tail of `tiles` tiles may be split: the workspace is there and holds the
+// partial tiles.
+inline bool tail_fits(int64_t tiles, int64_t K, int bm, int cus, const SmallSpace& ws) {
+  const int rest = (int)(tiles % cus);
+  return ws.words > 0 && (int64_t)rest * (tail_parts(rest, K, bm, cus, false) - 1) * bm * 256 * 4 <= ws.tile_bytes;
+}
+
 // ---------------------------------------------------------------------------
 // Which of the two
 // ---------------------------------------------------------------------------
@@ -180,9 +187,8 @@ inline int tail_parts(int R, int64_t K, int bm, int n_cons, bool reduce) {
 inline bool gemm_runs_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int cus, const SmallSpace& ws,
                             GemmSmallPlan* plan) {
   if (!plan_gemm_small(M, N, K, lda, ldb, cus, ws, {-1, 0}, plan)) return false;
-  const bool split = ws.words > 0;
   const int64_t t256 = M % 256 ? 0 : (M / 256) * (N / 256);
-  if (2 * t256 > cus && persistent_cost(t256, K, cus, split) <= plan->us) return false;
+  if (2 * t256 > cus && persistent_cost(t256, K, cus, tail_fits(t256, K, 256, cus, ws)) <= plan->us) return false;
   // An odd number of 128-row blocks, a last round of 128 x 256 tiles that can be
   // split along K, and a K long enough for it (the more rounds, the less the
   // last one weighs): the persistent kernel.  us, its time against the small
@@ -194,7 +200,8 @@ inline bool gemm_runs_small(int64_t M, int64_t N, int64_t K, int64_t lda, int64_
   // Over 267 such shapes the choice costs 0.7 % in the mean, 2.2 % when the line
   // was at 320 tiles of K 4096 and more.
   const int64_t t128 = (M / 128) * (N / 256), rounds = t128 / cus, rest = t128 % cus;
-  return !(M % 256 && split && rounds && rest && 20 * rest <= 9 * cus && K >= 1000 * (rounds + 3));
+  return !(M % 256 && rounds && rest && 20 * rest <= 9 * cus && K >= 1000 * (rounds + 3) &&
+           tail_fits(t128, K, 128, cus, ws));
 }
 
 struct FusedPlan {

@@ -21,6 +21,11 @@ static const mk::SmallSpace kSpace[2] = {{0, 0}, {496, 256LL * 262144}};
 extern "C" {
 int n_tiles() { return sizeof mk::kTiles / sizeof mk::kTiles[0]; }
 int fold_only(int i) { return mk::kTiles[i].fold_only; }
+// a workspace that holds `tiles` partial tiles of 128 x 256
+int gemm_within(int64_t M, int64_t N, int64_t K, int64_t tiles) {
+  mk::GemmSmallPlan p = {};
+  return mk::gemm_runs_small(M, N, K, K, N, 256, {496, tiles * 131072}, &p);
+}
 // out: tile, workgroups, parts along K
 int gemm(int64_t M, int64_t N, int64_t K, int ws, int* out) {
   mk::GemmSmallPlan p = {};
@@ -48,6 +53,7 @@ def plans(tmp_path_factory):
                     str(d / "plans.cpp"), "-o", str(d / "plans.so")], check=True, capture_output=True)
     lib = C.CDLL(str(d / "plans.so"))
     i64, i32 = C.c_int64, C.c_int
+    lib.gemm_within.argtypes = [i64, i64, i64, i64]
     lib.gemm.argtypes = [i64, i64, i64, i32, C.c_void_p]
     lib.fused.argtypes = [i64, i64, i64, i32, i64, i32, i32, C.c_void_p]
     lib.parts.argtypes = [i32, i64, i32, i32, i32]
@@ -81,8 +87,12 @@ def test_small_gemm_shapes(plans):
 def test_odd_row_blocks(plans, M, N, K, persistent):
     """Odd numbers of 128-row blocks go to the persistent kernel where its last
     round is split along K and K is long for the number of rounds; without a
-    workspace there is no split."""
+    workspace, or with one that is a tile too small, there is no split."""
     assert _gemm(plans, M, N, K)[0] != bool(persistent) and _gemm(plans, M, N, K, ws=0)[0]
+    if persistent:
+        rest = M // 128 * (N // 256) % 256
+        tiles = rest * (plans.parts(rest, K, 128, 256, 0) - 1)
+        assert not plans.gemm_within(M, N, K, tiles) and plans.gemm_within(M, N, K, tiles - 1)
 
 
 def _blocks(world, rows, copies=1):
