@@ -232,7 +232,9 @@ typedef struct mk_gemm_ar_args {
   uint32_t* error_word;
   uint32_t* stage_counters;     /* [(world-1) * M/128] for producers == -1 */
   uint32_t* done_flags;         /* [(M/256) * (N/256)] or NULL */
-  void* split_ws;
+  void* split_ws;               /* as in mk_gemm_rs; also counts the parts of done_flags' tiles where
+                                   those are computed in smaller ones (a product of few tiles takes
+                                   longer with done_flags and no split_ws) */
   int64_t split_ws_bytes;
   /* Optional device word holding the epoch: when set, the launch reads the
    * epoch from it (never 0) instead of `epoch`, so a HIP graph that records
@@ -282,7 +284,9 @@ typedef struct mk_gemm_ar2_args {
   uint32_t* error_word;
   uint32_t* stage_counters;     /* [2 * (world-1) * (M/world)/128] */
   uint32_t* done_flags;         /* [(M/256) * (N/256)] or NULL */
-  void* split_ws;
+  void* split_ws;               /* as in mk_gemm_rs; also counts the parts of done_flags' tiles where
+                                   those are computed in smaller ones (a product of few tiles takes
+                                   longer with done_flags and no split_ws) */
   int64_t split_ws_bytes;
   const uint32_t* epoch_ptr;
 } mk_gemm_ar2_args;

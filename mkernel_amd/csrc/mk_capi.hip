@@ -188,11 +188,13 @@ int small_gemm(const mk_gemm_args* a, int cus, void* stream) {
 // Where that kernel would split its tail along K it runs, so that results do not
 // depend on how the blocks arrive.  Not for flags that someone else publishes:
 // those must be able to arrive while the launch waits.
-int small_fused(mk::GemmKParams& p, bool reduce, void* split_ws, int cus, void* stream, const char* where) {
+int small_fused(mk::GemmKParams& p, bool reduce, void* split_ws, int64_t split_ws_bytes, int cus, void* stream,
+                const char* where) {
   if (p.sk_split > 1) return kNoSmallPlan;
   // the parts of a done flag's tile are counted in the workspace and stored
   // through a buffer window of up to 128 rows
-  const bool flags = !p.ar_done || (split_ws && (int64_t)p.rs_own_rows / 256 * p.tiles_n <= kSmallWords &&
+  const bool flags = !p.ar_done || (split_ws && split_ws_bytes >= kSplitFlagBytes &&
+                                    (int64_t)p.rs_own_rows / 256 * p.tiles_n <= kSmallWords &&
                                     128LL * p.ldc * 2 < (1LL << 31));
   const mk::FusedPlan f = mk::plan_fused(p.M, p.N, p.K, p.lda, p.ldb, cus, {reduce ? p.rs_npeers : -1, p.rs_own_rows},
                                          p.st_nblocks, p.st_src2 != nullptr, flags);
@@ -465,7 +467,7 @@ int prepare_ag(const mk_ag_gemm_args* a, void* stream, mk::GemmKParams& p, int* 
 
 int launch_ag(mk::GemmKParams& p, int costage, int small_cus, void* stream) {
   if (small_cus) {
-    const int rc = small_fused(p, false, nullptr, small_cus, stream, "mk_ag_gemm launch");
+    const int rc = small_fused(p, false, nullptr, 0, small_cus, stream, "mk_ag_gemm launch");
     if (rc != kNoSmallPlan) return rc;
   }
   hipError_t e = costage ? mk::launch_gemm_costaged(p, mk::kEpiStore, costage, static_cast<hipStream_t>(stream))
@@ -609,7 +611,7 @@ int rs_launch(const mk_gemm_rs_args* a, const void* peer_reduced, uint16_t* full
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, fn)) return rc;
   plan_split(p, bm, a->split_ws, a->split_ws_bytes, 256, true);
   if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
-    const int rc = small_fused(p, true, a->split_ws, d.cus, stream, fn);
+    const int rc = small_fused(p, true, a->split_ws, a->split_ws_bytes, d.cus, stream, fn);
     if (rc != kNoSmallPlan) return rc;
   }
   hipError_t e = costage_waves ? mk::launch_gemm_costaged(p, mk::kEpiReduce, costage_waves * total,
@@ -724,7 +726,7 @@ int mk_gemm_ar(const mk_gemm_ar_args* a, void* stream) {
   if (int rc = check_ws(a->split_ws, a->split_ws_bytes, "mk_gemm_ar")) return rc;
   plan_split(p, bm, a->split_ws, a->split_ws_bytes, 256, true);
   if (a->num_cus == 0 && !(p.rs_flags && !coop) && !costage_waves) {  // staged by this call, or not gated at all
-    const int rc = small_fused(p, true, a->split_ws, d.cus, stream, "mk_gemm_ar launch");
+    const int rc = small_fused(p, true, a->split_ws, a->split_ws_bytes, d.cus, stream, "mk_gemm_ar launch");
     if (rc != kNoSmallPlan) return rc;
   }
   hipError_t e = costage_waves ? mk::launch_gemm_costaged(p, mk::kEpiReduce, costage_waves * total,

@@ -146,7 +146,8 @@ __device__ __forceinline__ void part_done(const GemmSmallParams& p, int row, int
 }
 
 template <class C, bool REDUCE>
-__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(1, C::WAVES_PER_SIMD))) void gemm_small_kernel(GemmSmallParams p) {
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(1, C::WAVES_PER_SIMD)))
+void gemm_small_kernel(GemmSmallParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / C::WN, wn = wave % C::WN;

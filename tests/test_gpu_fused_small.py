@@ -138,7 +138,8 @@ def test_ar_two_shot_small(dev, world, rank, M, N, K):
 def test_done_flags_come_from_the_tiles(dev, world, M, N, K, two_shot):
     """Done flags are published by the launch that folds the tiles, not by one
     behind it, under several epochs (the parts are counted in the workspace,
-    which is left zeroed), and without a workspace too."""
+    which is left zeroed), and without a workspace, or with one too small for
+    its words, too: then nothing behind it is touched."""
     print(f"done flags world={world} M={M} N={N} K={K} two_shot={two_shot}", flush=True)
     A, B = wl.randn_bf16((M, K), 8, K ** -0.5).to(dev), wl.randn_bf16((K, N), 9, K ** -0.5).to(dev)
     rows, rank = (M // world, world - 1) if two_shot else (M, 0)
@@ -161,15 +162,16 @@ def test_done_flags_come_from_the_tiles(dev, world, M, N, K, two_shot):
 
     lo, hi = rank * rows // 256 * (N // 256), (rank + 1) * rows // 256 * (N // 256)
     outs = []
-    for split in (ws, ws, False):
+    little = torch.full((4096,), 7, dtype=torch.uint8, device=dev)
+    for split in (ws, ws, False, little[:1024]):
         epoch += 1
         done.zero_()
         call(split, done, epoch_ptr=epoch)
         torch.cuda.synchronize()
         assert bool((done[lo:hi] == epoch).all()) and int((done != 0).sum()) == hi - lo
-        assert not bool(ws[:4096].any())
+        assert not bool(ws[:4096].any()) and bool((little == 7).all())
         outs.append(C.clone())
-    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
     assert _graph_nodes(lambda: call(ws, done, epoch_ptr=epoch)) == _graph_nodes(lambda: call(ws, None, epoch_ptr=epoch))
 
 
