@@ -56,10 +56,11 @@ constexpr TileCost kTiles[] = {
     {64, 64, 5, true, 0.8, 2.2, 0.300, 0.0, 0.31, 0.155, 7.0},
 };
 // fold_only, the 32 KB ring of the last: its many workgroups hide a fold's loads
-// (whole ReduceScatters, against the 128 x 128 tiles at 128 KB: 4096x4096x256 of
-// world 16 41 us / 44, 2048x2304x32 of world 8 16.6 / 18.1, 4096x2048x128 of
-// world 16 24.7 / 27.4), but a plain product of tall tiles thrashes L2 with them
-// (5504x768x896 18.5 us, 14.5 with the 128 x 128 tiles at 64 KB).
+// (whole ReduceScatters, against the 128 x 128 tiles at 64 KB: 4096x4096x256 of
+// world 16 40.4 us / 44.2, 2048x2304x32 of world 8 16.0 / 17.6, 4096x2048x128 of
+// world 16 23.4 / 27.6; the 64 x 64 tiles at 48 KB are level with it), but a plain
+// product of tall tiles thrashes L2 with them (5504x768x896 18.5 us, 14.5 with
+// the 128 x 128 tiles at 64 KB).
 
 inline double rounds_cost(const TileCost& c, int64_t g, double stages, int cus) {
   const int64_t full = (int64_t)c.per_cu * cus;

@@ -164,6 +164,28 @@ __device__ __forceinline__ void store_rows(uint16_t* base, int64_t ldc, f32x16 (
   }
 }
 
+// x += 8 columns of n <= G partials, in order, their loads in flight together
+// (indices clamped to the last, so no branch splits the loads; the empty asm
+// keeps the compiler from moving each load to its adds, one latency after
+// another: ReduceScatter 4096x4096x256 of world 16 took 49.5 us so, 37.9 with
+// it; groups of 8 for all but the first peers made one peer's fold 5 % slower).
+template <int G>
+__device__ __forceinline__ void fold_group(const uint16_t* src, int64_t peer_stride, int n, float (&x)[8]) {
+  uint4 v[G];
+#pragma unroll
+  for (int u = 0; u < G; ++u) v[u] = *reinterpret_cast<const uint4*>(src + (int64_t)min(u, n - 1) * peer_stride);
+#pragma unroll
+  for (int u = 0; u < G; ++u) asm volatile("" : "+v"(v[u].x), "+v"(v[u].y), "+v"(v[u].z), "+v"(v[u].w));
+#pragma unroll
+  for (int u = 0; u < G; ++u)
+    if (u < n) {
+      x[0] += bf16_lo(v[u].x); x[1] += bf16_hi(v[u].x);
+      x[2] += bf16_lo(v[u].y); x[3] += bf16_hi(v[u].y);
+      x[4] += bf16_lo(v[u].z); x[5] += bf16_hi(v[u].z);
+      x[6] += bf16_lo(v[u].w); x[7] += bf16_hi(v[u].w);
+    }
+}
+
 // Reduce epilogue of an owned tile, row-major: each 32-row block of the
 // wave's fp32 accumulators goes through the wave's LDS region (rows of WTN
 // fp32, pitch padded by 16 bytes) and comes back 8 columns per lane with
@@ -173,10 +195,12 @@ __device__ __forceinline__ void store_rows(uint16_t* base, int64_t ldc, f32x16 (
 // adds them in rank order in fp32
 // (deterministic, one rounding) and stores 16 bytes of the owned output.
 // In the accumulator layout every load and store instruction would touch
-// 32 rows with 8 bytes each.  FLAGGED: with p.done the output goes out write-
-// through (performed at agent scope once vmcnt says it is stored, the protocol
-// of copy_wt), for a flag that needs no L2 write-back.
-template <class C, int kPeers = 4, bool FLAGGED = false, class P>
+// 32 rows with 8 bytes each.  SMALL (the small-tile kernel; the 256-row kernel
+// has no registers left for it): the last peers by fold_group, and with p.done
+// the output goes out write-through (performed at agent scope once vmcnt says
+// it is stored, the protocol of copy_wt), for a flag that needs no L2
+// write-back.
+template <class C, int kPeers = 4, bool SMALL = false, class P>
 __device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::FN], int lrow0, int col0,
                                             char* smem, int wave, int lane) {
   constexpr int PITCH = C::WTN * 4 + 16;  // bytes per LDS row (fp32)
@@ -225,7 +249,12 @@ __device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::
           x[6] += bf16_lo(v[u].w); x[7] += bf16_hi(v[u].w);
         }
       }
-      if (q < np) {
+      if constexpr (SMALL) {
+        const uint16_t* rest = src + q * peer_stride;
+        if (np - q > 4) fold_group<kPeers>(rest, peer_stride, np - q, x);
+        else if (np - q > 1) fold_group<4>(rest, peer_stride, np - q, x);
+        else if (np - q == 1) fold_group<1>(rest, peer_stride, 1, x);
+      } else if (q < np) {
         // the last np - q peers as one more group in flight (indices
         // clamped to the last peer, so no branch splits the loads)
         uint4 v[kPeers];
@@ -244,7 +273,7 @@ __device__ __forceinline__ void reduce_rows(const P& p, f32x16 (&acc)[C::FM][C::
       uint4 o;
       o.x = pack_bf16x2(x[0], x[1]); o.y = pack_bf16x2(x[2], x[3]);
       o.z = pack_bf16x2(x[4], x[5]); o.w = pack_bf16x2(x[6], x[7]);
-      if constexpr (FLAGGED)
+      if constexpr (SMALL)
         if (p.done) {
           __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{o.x, o.y, o.z, o.w}, out,
                                                  (int)(((i * 32 + row) * p.ldc + cc * 8) * 2), 0, 0x10 /* SC1 */);
